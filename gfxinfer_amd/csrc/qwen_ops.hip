@@ -12,6 +12,7 @@
 #include <utility>
 
 #include "common.hpp"
+#include "prefill.hpp"
 
 namespace gfx950 {
 namespace {
@@ -1530,6 +1531,16 @@ extern "C" int32_t gfxinfer_launch_mtp_input_quantize_i4_from_keys(
 
 // ---- SwiGLU -----------------------------------------------------------------
 
+namespace gfx950 {
+int32_t silu_multiply_quantize_rows(const float* gate, const float* up, uint8_t* codes, uint16_t* scales,
+                                    std::size_t columns, uint32_t rows, hipStream_t stream) {
+  const auto total = static_cast<uint32_t>(columns / 128 * rows);
+  hipLaunchKernelGGL(silu_multiply_kernel<true>, dim3((total + 3) / 4), dim3(256), 0, stream, gate, up, nullptr,
+                     codes, reinterpret_cast<__half*>(scales), static_cast<uint32_t>(columns), total);
+  return launch_status("fused SiLU/A4 quantization launch failed");
+}
+}  // namespace gfx950
+
 extern "C" int32_t gfxinfer_launch_silu_multiply_quantize_i4(const float* gate, const float* up,
                                                              uint8_t* packed_output,
                                                              uint16_t* scales,
@@ -1540,12 +1551,8 @@ extern "C" int32_t gfxinfer_launch_silu_multiply_quantize_i4(const float* gate, 
       elements_per_row > (1u << 30)) {
     return fail(GFXI_INVALID_ARGUMENT, "invalid fused SiLU/A4 quantization arguments");
   }
-  const auto columns = static_cast<uint32_t>(elements_per_row);
-  const uint32_t total = columns / 128 * batch;
-  hipLaunchKernelGGL(silu_multiply_kernel<true>, dim3((total + 3) / 4), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), gate, up, nullptr, packed_output,
-                     reinterpret_cast<__half*>(scales), columns, total);
-  return launch_status("fused SiLU/A4 quantization launch failed");
+  return silu_multiply_quantize_rows(gate, up, packed_output, scales, elements_per_row, batch,
+                                     static_cast<hipStream_t>(stream));
 }
 
 extern "C" int32_t gfxinfer_launch_silu_multiply(const float* gate, const float* up,
@@ -1641,6 +1648,24 @@ extern "C" int32_t gfxinfer_launch_gdn_recurrent_decode_block(
   return launch_status("block GDN output norm launch failed");
 }
 
+namespace {
+int32_t launch_gdn_output_quantize(const float* mixed, const float* z, const uint16_t* norm_weight, uint16_t* output,
+                                   uint8_t* codes, uint16_t* scales, uint32_t tokens, uint32_t value_heads,
+                                   hipStream_t stream) {
+  const uint32_t total = tokens * value_heads;
+  hipLaunchKernelGGL(gdn_output_kernel<true>, dim3((total + 3) / 4), dim3(256), 0, stream, mixed, z, norm_weight,
+                     reinterpret_cast<__half*>(output), codes, reinterpret_cast<__half*>(scales), value_heads, total);
+  return launch_status("GDN output/A4 launch failed");
+}
+}  // namespace
+
+namespace gfx950 {
+int32_t gdn_output_quantize_rows(const float* mixed, const float* z, const uint16_t* norm_weight, uint8_t* codes,
+                                 uint16_t* scales, uint32_t rows, uint32_t value_heads, hipStream_t stream) {
+  return launch_gdn_output_quantize(mixed, z, norm_weight, nullptr, codes, scales, rows, value_heads, stream);
+}
+}  // namespace gfx950
+
 extern "C" int32_t gfxinfer_launch_gdn_output_quantize_i4(
     const float* mixed, const float* projected_z, const uint16_t* bf16_norm_weight,
     uint16_t* output, uint8_t* packed_output, uint16_t* scales, uint32_t batch,
@@ -1650,12 +1675,8 @@ extern "C" int32_t gfxinfer_launch_gdn_output_quantize_i4(
       value_heads == 0 || head_size != kGdnD) {
     return fail(GFXI_INVALID_ARGUMENT, "invalid GDN output/A4 arguments");
   }
-  const uint32_t total = batch * value_heads;
-  hipLaunchKernelGGL(gdn_output_kernel<true>, dim3((total + 3) / 4), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), mixed, projected_z, bf16_norm_weight,
-                     reinterpret_cast<__half*>(output), packed_output, reinterpret_cast<__half*>(scales),
-                     value_heads, total);
-  return launch_status("GDN output/A4 launch failed");
+  return launch_gdn_output_quantize(mixed, projected_z, bf16_norm_weight, output, packed_output, scales, batch,
+                                    value_heads, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int32_t gfxinfer_launch_gdn_recurrent_window(

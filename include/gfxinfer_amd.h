@@ -220,6 +220,19 @@ int32_t gfxinfer_debug_gemm_family(int32_t family, int32_t format, const uint8_t
                                    size_t rows, size_t columns, uint32_t batch, uint32_t splits,
                                    void* stream);
 
+/* Test and bench hook, no reference counterpart: the GEMM of the session's wide prefill pass
+ * (prompts of 65 tokens or more, gfxinfer_session_prefill) on its own.  Arguments and
+ * results as gfxinfer_launch_gfx950_i4_gemm_split (fp32 planes, or fp16 [tokens][rows] with
+ * half_output != 0 and one split) at any token count; the workspace (16-byte aligned) holds
+ * the expanded activations.  Bit-identical to the block launchers. */
+size_t gfxinfer_debug_gemm_prefill_workspace_bytes(size_t columns, uint32_t tokens);
+int32_t gfxinfer_debug_gemm_prefill(int32_t format, const uint8_t* tiled_weights,
+                                    const uint16_t* tiled_weight_scales,
+                                    const uint8_t* packed_activations,
+                                    const uint16_t* activation_scales, void* output,
+                                    int32_t half_output, size_t rows, size_t columns, uint32_t tokens,
+                                    uint32_t splits, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Calibration: a plain streaming read of `bytes` from `data` (16-byte aligned,
  * a nonzero multiple of 16) by `workgroups` x 256 lanes, so that a weight-streaming
  * kernel's time can be set beside what one launch reading the same bytes takes on the

@@ -292,8 +292,8 @@ int32_t gfxinfer_session_set_layer_trace(gfxinfer_session* session, void* device
 
 /* Chunked prefill.  The reference prefills a prompt with one greedy_step per token and,
  * when MTP is on, an mtp_draft per token from the second on (cli/main.cpp:1055-1069);
- * this runs the target over the prompt in blocks of up to 32 tokens and, with
- * sync_mtp != 0, advances the MTP K/V cache over the same positions in batches (entry j
+ * this runs the target over the prompt in wide passes (65 to 512 tokens) and blocks of up
+ * to 32 tokens and, with sync_mtp != 0, advances the MTP K/V cache over the same positions in batches (entry j
  * from token j + 1 and the target's hidden state at position j), leaving the target,
  * GDN, KV and MTP cache state and the positions as that serial loop leaves them.
  * *next_token = the greedy token after the last prompt token.  Requires a fresh
