@@ -40,6 +40,26 @@ int32_t prefill_gemm(int32_t format, const PrefillMatrix* matrices, std::size_t 
                      const PrefillOperand& in, std::size_t columns, uint32_t tokens, uint32_t splits,
                      bool half_output, hipStream_t stream);
 
+// gfxinfer_launch_gdn_conv_window over any number of tokens, without logs.  Rows 16-byte
+// aligned; conv and recurrent states are not updated in place.
+struct GdnPrefillPass {
+  const float* projected;         // [tokens][channels]
+  const uint16_t* conv_weight;    // bf16 [channels][4]
+  const uint16_t* conv_initial;   // fp16 [channels][4]
+  uint16_t* conv_final;
+  const float* a;                 // [tokens][value_heads]
+  const float* b;
+  const uint16_t* a_log;          // bf16 [value_heads]
+  const uint16_t* dt_bias;
+  float* convolved;               // scratch [tokens][channels]
+  float* gates;                   // scratch [2][tokens][value_heads]
+  const float* initial_state;     // [value_heads][128][128]
+  float* final_state;
+  float* mixed;                   // [tokens][value_heads * 128]
+  uint32_t tokens, key_heads, value_heads;
+};
+int32_t gdn_prefill(const GdnPrefillPass& pass, hipStream_t stream);
+
 // The block launchers' kernels over any number of rows.
 int32_t quantize_activation_rows(const uint16_t* input, uint8_t* codes, uint16_t* scales, std::size_t columns,
                                  uint32_t rows, hipStream_t stream);

@@ -13,12 +13,12 @@
 #include <utility>
 
 #include "common.hpp"
+#include "gemm_common.hpp"
 #include "prefill.hpp"
 
 namespace gfx950 {
 namespace {
 
-using u32x4 = unsigned __attribute__((ext_vector_type(4)));
 using f32x4 = float __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float silu(float x) { return x / (1.0F + expf(-x)); }
@@ -987,6 +987,202 @@ __global__ __launch_bounds__(kWindowThreads) void gdn_window_kernel(GdnWindowArg
   }
 }
 
+// ---------------------------------------------------------------------------
+// GDN over a prefill pass (more than 32 tokens): gdn_window_kernel's arithmetic in two
+// launches.  In windows, every workgroup of a key head convolves and normalizes that head's
+// query and key channels again (16 times at 32 value heads) while the recurrence waits, and
+// the state goes to memory and back every 32 tokens; here the convolution runs once over
+// all tokens, in parallel, and one workgroup per (head, 16 columns) keeps its state in
+// registers from the first token to the last.
+// ---------------------------------------------------------------------------
+
+struct GdnPrefillArgs {
+  const float* projected;       // [T][C] fp32 (q heads | k heads | v heads)
+  const uint16_t* conv_weight;  // bf16 [C][4]
+  const __half* conv_initial;   // [C][4]
+  __half* conv_final;           // [C][4]
+  const float* a;               // [T][Hv]
+  const float* b;               // [T][Hv]
+  const uint16_t* a_log;        // bf16 [Hv]
+  const uint16_t* dt_bias;      // bf16 [Hv]
+  float* convolved;             // [T][C]: normalized queries (scaled) and keys, values
+  float* gates;                 // decay [T][Hv], then beta [T][Hv]
+  const float* initial;         // [Hv][D][D]
+  float* final_state;           // [Hv][D][D]
+  float* mixed;                 // [T][Hv*D]
+  uint32_t tokens, key_heads, value_heads;
+};
+
+// One wave per (128-channel head, run of eight tokens): the four taps of eight tokens are
+// eleven rows, loaded once.  Bound by memory: reads and writes [T][C] fp32 once.
+constexpr unsigned kGdnRun = 8;
+
+__global__ __launch_bounds__(256) void gdn_prefill_conv_kernel(GdnPrefillArgs g) {
+  constexpr unsigned D = kGdnD;
+  const uint32_t heads = 2 * g.key_heads + g.value_heads;
+  const uint32_t linear = blockIdx.x * 4u + (threadIdx.x >> 6);
+  const uint32_t head = linear % heads, t0 = linear / heads * kGdnRun;
+  if (t0 >= g.tokens) return;  // wave-uniform
+  const unsigned lane = threadIdx.x & 63u;
+  const std::size_t C = static_cast<std::size_t>(heads) * D;
+  const std::size_t c = static_cast<std::size_t>(head) * D + 2 * lane;  // this lane's two channels
+  float2 in[kGdnRun + 3];
+#pragma unroll
+  for (unsigned r = 0; r < kGdnRun + 3; ++r) {  // rows past the ends: a valid row, not used
+    const uint32_t row = t0 + r < 3u ? 0u : min(t0 + r - 3u, g.tokens - 1u);
+    in[r] = *reinterpret_cast<const float2*>(g.projected + static_cast<std::size_t>(row) * C + c);
+  }
+  const u32x4 taps = *reinterpret_cast<const u32x4*>(g.conv_weight + c * 4);      // 2 channels x 4 bf16
+  const u32x4 before = *reinterpret_cast<const u32x4*>(g.conv_initial + c * 4);   // 2 channels x 4 fp16
+  float w[2][4];
+  __half x[kGdnRun + 3][2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+#pragma unroll
+    for (int tap = 0; tap < 4; ++tap) {
+      w[e][tap] = bf16_to_float(static_cast<uint16_t>(taps[2 * e + tap / 2] >> (16 * (tap % 2))));
+    }
+  }
+#pragma unroll
+  for (unsigned r = 0; r < kGdnRun + 3; ++r) {
+    x[r][0] = to_half(in[r].x);
+    x[r][1] = to_half(in[r].y);
+    if (r < 3u && t0 == 0) {  // the inputs before the first token: taps 1 .. 3 of the state
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        x[r][e] = __ushort_as_half(static_cast<unsigned short>(before[2 * e + (r + 1) / 2] >> (16 * ((r + 1) % 2))));
+      }
+    }
+  }
+  const bool key_side = head < 2 * g.key_heads, query = head < g.key_heads;
+  const float query_scale = 0.08838834764831845F;  // 1/sqrt(128), qwen_ops.hip:325
+#pragma unroll
+  for (unsigned t = 0; t < kGdnRun; ++t) {
+    if (t0 + t >= g.tokens) break;  // wave-uniform
+    float y[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      float conv = 0.0F;
+#pragma unroll
+      for (int tap = 0; tap < 4; ++tap) conv = fmaf(__half2float(x[t + tap][e]), w[e][tap], conv);
+      y[e] = __half2float(to_half(silu(conv)));
+    }
+    if (key_side) {
+      float inverse = rsqrtf(wave_sum(y[0] * y[0] + y[1] * y[1]) + 1.0e-6F);
+      if (query) inverse = inverse * query_scale;
+      y[0] = y[0] * inverse;
+      y[1] = y[1] * inverse;
+    }
+    *reinterpret_cast<float2*>(g.convolved + static_cast<std::size_t>(t0 + t) * C + c) = float2{y[0], y[1]};
+  }
+  // The last run's rows end with the pass's last four inputs: the final conv state.
+  if (t0 + kGdnRun >= g.tokens) {
+    const unsigned live = g.tokens - t0;  // 1 .. 8 tokens: inputs T - 4 .. T - 1 are rows live - 1 .. live + 2
+#pragma unroll
+    for (unsigned k = 1; k <= kGdnRun; ++k) {
+      if (k != live) continue;
+      uint32_t bits[4];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          bits[2 * e + p] = __half_as_ushort(x[k - 1 + 2 * p][e]) |
+                            (static_cast<uint32_t>(__half_as_ushort(x[k + 2 * p][e])) << 16);
+        }
+      }
+      *reinterpret_cast<u32x4*>(g.conv_final + c * 4) = u32x4{bits[0], bits[1], bits[2], bits[3]};
+    }
+  }
+  // Decay and beta of the run's tokens (qwen_ops.hip:342-349), one lane each.
+  if (!key_side && lane < kGdnRun && t0 + lane < g.tokens) {
+    const uint32_t h = head - 2 * g.key_heads;
+    const std::size_t at = static_cast<std::size_t>(t0 + lane) * g.value_heads + h;
+    const float a_value = g.a[at] + bf16_to_float(g.dt_bias[h]);
+    const float softplus = a_value > 20.0F ? a_value : log1pf(expf(a_value));
+    const float gate = -expf(bf16_to_float(g.a_log[h])) * softplus;
+    g.gates[at] = expf(gate);
+    g.gates[static_cast<std::size_t>(g.tokens) * g.value_heads + at] = 1.0F / (1.0F + expf(-g.b[at]));
+  }
+}
+
+// Workgroup = (value head, 16 state columns), four waves as in gdn_recurrent_kernel; the
+// operands of 32 tokens at a time come by DMA into one of two LDS sides while the other
+// side's tokens are scanned.  Bound by the recurrence's chain (gdn_scan).  509 tokens at 32
+// value heads: convolution 12.5 us and scan 87 us, against 16 windows of 12.8 us.
+constexpr unsigned kScanTokens = 32;
+struct GdnScanSide {
+  float keys[kScanTokens][kGdnD];
+  float queries[kScanTokens][kGdnD];
+  float values[kScanTokens][kGdnCols];
+  float decay[kScanTokens];
+  float beta[kScanTokens];
+};
+
+__global__ __launch_bounds__(256) void gdn_prefill_scan_kernel(GdnPrefillArgs g) {
+  constexpr unsigned D = kGdnD;
+  // Two objects, so that the compiler sees which side a DMA writes.
+  __shared__ __align__(16) GdnScanSide side0, side1;
+  const unsigned blocks_per_head = D / kGdnCols;
+  const unsigned h = blockIdx.x / blocks_per_head, cb = blockIdx.x - h * blocks_per_head;
+  const unsigned kh = h / (g.value_heads / g.key_heads);
+  const unsigned lane = threadIdx.x & 63u;
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t T = g.tokens, Hv = g.value_heads;
+  const uint32_t row = (2 * g.key_heads + Hv) * D * 4u;  // bytes of a convolved row
+  const auto convolved = buffer(g.convolved, T * row);
+  const auto gates = buffer(g.gates, 2u * T * Hv * 4u);
+  auto load = [&](GdnScanSide& side, unsigned t0) __attribute__((always_inline)) {
+    // Two rows of 512 bytes per instruction; rows past the last token repeat it, unused.
+#pragma unroll
+    for (unsigned p = 0; p < kScanTokens / 8; ++p) {
+      const unsigned pair = (p * 4u + wave) * 2u;
+      const unsigned at = min(t0 + pair + lane / 32u, T - 1u) * row + lane % 32u * 16u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(convolved, (lds_void*)&side.queries[pair][0], 16, at, kh * D * 4u, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(convolved, (lds_void*)&side.keys[pair][0], 16, at,
+                                               (g.key_heads + kh) * D * 4u, 0, 0);
+    }
+    if (wave < 2) {
+      const unsigned t = wave * 16u + lane / 4u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(convolved, (lds_void*)&side.values[wave * 16u][0], 16,
+                                               min(t0 + t, T - 1u) * row + lane % 4u * 16u,
+                                               ((2 * g.key_heads + h) * D + cb * kGdnCols) * 4u, 0, 0);
+    } else if (wave == 2) {  // decay, then beta
+      const unsigned t = min(t0 + lane % 32u, T - 1u);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(gates, (lds_void*)&side.decay[0], 4,
+                                               ((lane < 32u ? 0u : T) + t) * Hv * 4u + h * 4u, 0, 0, 0);
+    }
+  };
+  // Every wave's DMA has arrived: vector-memory operations complete in issue order, and a
+  // side whose DMA is followed by another scan holds 32 tokens, whose two stores are younger.
+  auto arrived = [&](auto younger) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(younger)::value) : "memory");
+  };
+  load(side0, 0);
+  const unsigned ks = lane & 15u;                // rows ks*8 .. ks*8+7
+  const unsigned col = wave * 4u + (lane >> 4);  // column within the block
+  const std::size_t out_column = static_cast<std::size_t>(h) * D + cb * kGdnCols + col;
+  const std::size_t value_elements = static_cast<std::size_t>(Hv) * D;
+  const std::size_t state = static_cast<std::size_t>(h) * D * D + cb * kGdnCols + col;
+  float S[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) S[i] = g.initial[state + static_cast<std::size_t>(ks * 8 + i) * D];
+  arrived(std::integral_constant<int, 0>{});
+  auto scan = [&](GdnScanSide& here, GdnScanSide& other, unsigned t0) __attribute__((always_inline)) {
+    if (t0 + kScanTokens < T) load(other, t0 + kScanTokens);
+    gdn_scan(S, here.keys, here.queries, here.values, here.decay, here.beta, min(kScanTokens, T - t0), ks, col,
+             g.mixed + static_cast<std::size_t>(t0) * value_elements, nullptr, value_elements, out_column);
+    static_assert(kScanTokens == 32, "two stores of sixteen tokens");
+    arrived(std::integral_constant<int, 2>{});
+  };
+  for (unsigned t0 = 0; t0 < T; t0 += 2 * kScanTokens) {
+    scan(side0, side1, t0);
+    if (t0 + kScanTokens >= T) break;
+    scan(side1, side0, t0 + kScanTokens);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) g.final_state[state + static_cast<std::size_t>(ks * 8 + i) * D] = S[i];
+}
+
 // Head RMSNorm * weight * SiLU(z) (qwen_ops.hip:386-409) of the mixed output,
 // optionally followed by the A4 quantizer (a head is exactly one 128 group).
 // One wave per (token, value head).
@@ -1711,6 +1907,21 @@ int32_t launch_gdn_output_quantize(const float* mixed, const float* z, const uin
 }  // namespace
 
 namespace gfx950 {
+int32_t gdn_prefill(const GdnPrefillPass& p, hipStream_t stream) {
+  if (p.tokens == 0 || p.key_heads == 0 || p.value_heads % p.key_heads != 0 ||
+      static_cast<uint64_t>(p.tokens) * (2 * p.key_heads + p.value_heads) * kGdnD * 4u > 0x7fffffffu) {
+    return fail(GFXI_INVALID_ARGUMENT, "invalid GDN prefill arguments");
+  }
+  const GdnPrefillArgs g{p.projected, p.conv_weight, reinterpret_cast<const __half*>(p.conv_initial),
+                         reinterpret_cast<__half*>(p.conv_final), p.a, p.b, p.a_log, p.dt_bias, p.convolved, p.gates,
+                         p.initial_state, p.final_state, p.mixed, p.tokens, p.key_heads, p.value_heads};
+  const uint32_t waves = (2 * p.key_heads + p.value_heads) * ((p.tokens + kGdnRun - 1) / kGdnRun);
+  hipLaunchKernelGGL(gdn_prefill_conv_kernel, dim3((waves + 3) / 4), dim3(256), 0, stream, g);
+  if (const int32_t s = launch_status("GDN prefill convolution launch failed"); s != GFXI_OK) return s;
+  hipLaunchKernelGGL(gdn_prefill_scan_kernel, dim3(p.value_heads * (kGdnD / kGdnCols)), dim3(256), 0, stream, g);
+  return launch_status("GDN prefill scan launch failed");
+}
+
 int32_t gdn_output_quantize_rows(const float* mixed, const float* z, const uint16_t* norm_weight, uint8_t* codes,
                                  uint16_t* scales, uint32_t rows, uint32_t value_heads, hipStream_t stream) {
   return launch_gdn_output_quantize(mixed, z, norm_weight, nullptr, codes, scales, rows, value_heads, stream);

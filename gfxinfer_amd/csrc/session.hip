@@ -202,6 +202,7 @@ struct gfxinfer_session {
   uint16_t* wide_scales{};
   float2* wide_meta{};
   float *wide_main{}, *wide_z{}, *wide_a{}, *wide_b{}, *wide_k{}, *wide_v{}, *wide_mixed{};
+  float *wide_convolved{}, *wide_gates{};
   float *wide_update{}, *wide_gate{}, *wide_up{};
 
   std::array<Graph, 2> graphs{};
@@ -544,9 +545,10 @@ struct gfxinfer_session {
 
   // ---- wide prefill pass --------------------------------------------------------
   // The layer block over T > 32 tokens: the block kernels' arithmetic value for value (the
-  // GEMM in prefill_gemm.hip; the others are the block launchers' kernels over more rows,
-  // or, for the attention and the GDN windows, their launches one 32-token block after the
-  // other), so every state, cache and hidden row equals the block-by-block pass.
+  // GEMM in prefill_gemm.hip and the GDN pass in qwen_ops.hip; the others are the block
+  // launchers' kernels over more rows, or, for the attention, its launches one 32-token
+  // block after the other), so every state, cache and hidden row equals the block-by-block
+  // pass.
 
   // A4 codes and scales in wide_codes / wide_scales -> the GEMM's operand.
   int32_t wide_operand(std::size_t columns, unsigned T, PrefillOperand& out) {
@@ -605,19 +607,12 @@ struct gfxinfer_session {
       }
     } else {
       GFXI_TRY(wide_gemm({{&L.qkv, wide_main}, {&L.z, wide_z}, {&L.a, wide_a}, {&L.b, wide_b}}, in, T));
-      // Window after window, the states going back and forth between the two buffers.
-      uint16_t* conv[2] = {conv_states + L.state_index * conv_state_elements(),
-                           conv_snapshot + L.state_index * conv_state_elements()};
-      float* state[2] = {gdn_states + L.state_index * gdn_state_elements(),
-                         gdn_snapshot + L.state_index * gdn_state_elements()};
-      for (unsigned a = 0, i = 0; a < T; a += kMaxBlock, i ^= 1u) {
-        GFXI_TRY(gfxinfer_launch_gdn_conv_window(
-            wide_main + a * channels, L.conv, conv[i], conv[i ^ 1u], nullptr,
-            wide_a + a * spec.gdn_value_head_count, wide_b + a * spec.gdn_value_head_count, L.a_log, L.dt_bias,
-            state[i], state[i ^ 1u], wide_mixed + a * gdn_value, nullptr, nullptr, nullptr,
-            std::min(kMaxBlock, T - a), spec.gdn_key_head_count, spec.gdn_value_head_count, spec.gdn_head_size,
-            stream));
-      }
+      // As one window: from the states into the snapshot buffers, swapped after the pass.
+      const std::size_t conv = L.state_index * conv_state_elements(), state = L.state_index * gdn_state_elements();
+      GFXI_TRY(gdn_prefill({wide_main, L.conv, conv_states + conv, conv_snapshot + conv, wide_a, wide_b, L.a_log,
+                            L.dt_bias, wide_convolved, wide_gates, gdn_states + state, gdn_snapshot + state, wide_mixed,
+                            T, spec.gdn_key_head_count, spec.gdn_value_head_count},
+                           stream));
       GFXI_TRY(gdn_output_quantize_rows(wide_mixed, wide_z, L.gdn_norm, wide_codes, wide_scales, T,
                                         spec.gdn_value_head_count, stream));
     }
@@ -697,11 +692,9 @@ struct gfxinfer_session {
     }
     GFXI_TRY(sync("prefill pass failed"));
     if (head) *next = host_result[last - 1];
-    if ((T + kMaxBlock - 1) / kMaxBlock % 2 != 0) {
-      std::swap(conv_states, conv_snapshot);
-      std::swap(gdn_states, gdn_snapshot);
-      parity = !parity;
-    }
+    std::swap(conv_states, conv_snapshot);
+    std::swap(gdn_states, gdn_snapshot);
+    parity = !parity;
     last_hidden = hidden_a + static_cast<std::size_t>(last - 1) * H;
     current_position += T;
     mtp_position += entries;
@@ -1261,6 +1254,8 @@ extern "C" int32_t gfxinfer_session_create(gfxinfer_model* model,
           {"wide_k", reinterpret_cast<void**>(&s->wide_k), W * s->kv_rows * 4},
           {"wide_v", reinterpret_cast<void**>(&s->wide_v), W * s->kv_rows * 4},
           {"wide_mixed", reinterpret_cast<void**>(&s->wide_mixed), W * s->gdn_value * 4},
+          {"wide_convolved", reinterpret_cast<void**>(&s->wide_convolved), W * s->channels * 4},
+          {"wide_gates", reinterpret_cast<void**>(&s->wide_gates), 2 * W * sp.gdn_value_head_count * 4},
           {"wide_update", reinterpret_cast<void**>(&s->wide_update), update_planes * W * s->H * 4},
           {"wide_gate", reinterpret_cast<void**>(&s->wide_gate), W * s->I * 4},
           {"wide_up", reinterpret_cast<void**>(&s->wide_up), W * s->I * 4},
