@@ -240,8 +240,10 @@ def _p(x) -> int | None:
 
 def _stream(stream) -> int | None:
     if stream is None:
+        # The handle of torch.cuda.current_stream() without its Stream object (2.8 us a call,
+        # as much as the launch itself).
         import torch
-        return torch.cuda.current_stream().cuda_stream
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
