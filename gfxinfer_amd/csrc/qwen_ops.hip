@@ -1240,12 +1240,14 @@ __global__ __launch_bounds__(256) void gdn_restore_conv_kernel(
   s[3] = w[3];
 }
 
-// Thread per four consecutive state columns of one row.
 // One workgroup per (layer, value head): the head's logged keys, deltas and decays of
-// the accepted tokens are staged in LDS once, then each thread replays them onto 16
+// the accepted tokens are staged in LDS once, then each thread replays them onto sixteen
 // four-column pieces of the 128 x 128 state (per element the same operations in token
-// order as the recurrence), so the logs cross the memory hierarchy once per head
-// instead of once per state piece.
+// order as the recurrence), so the logs cross the memory hierarchy once per head instead
+// of once per state piece.  A thread's pieces are the same four columns of four rows in
+// a row, four times over: a token costs it one read each of the deltas, the decay and the
+// keys per four pieces (reads per piece made the LDS the bound), and the four quarters of
+// the state, one after the other, overlap their stores with the next one's arithmetic.
 constexpr unsigned kRestoreThreads = 256;
 
 __global__ __launch_bounds__(kRestoreThreads) void gdn_restore_recurrent_kernel(
@@ -1254,18 +1256,24 @@ __global__ __launch_bounds__(kRestoreThreads) void gdn_restore_recurrent_kernel(
     uint32_t value_heads) {
   constexpr unsigned D = kGdnD;
   constexpr unsigned kPieces = D * D / 4 / kRestoreThreads;  // 16 f32x4 per thread
-  __shared__ float keys[kGdnMaxTokens][D];
-  __shared__ float deltas[kGdnMaxTokens][D];
+  constexpr unsigned kQuarters = kPieces / 4;
+  constexpr unsigned kRows = kRestoreThreads / (D / 4) * 4;  // rows per quarter
+  __shared__ __align__(16) float keys[kGdnMaxTokens][D];
+  __shared__ __align__(16) float deltas[kGdnMaxTokens][D];
   __shared__ float decays[kGdnMaxTokens];
   const unsigned layer = blockIdx.x / value_heads, h = blockIdx.x - layer * value_heads;
   const unsigned kh = h / (value_heads / key_heads);
   const unsigned tid = threadIdx.x;
   const std::size_t key_elements = static_cast<std::size_t>(key_heads) * D;
   const std::size_t value_elements = static_cast<std::size_t>(value_heads) * D;
-  f32x4* state = reinterpret_cast<f32x4*>(states + (static_cast<std::size_t>(layer) * value_heads + h) * D * D);
-  f32x4 S[kPieces];
+  const unsigned k0 = tid / (D / 4) * 4, v = tid % (D / 4) * 4;
+  f32x4* state = reinterpret_cast<f32x4*>(states + ((static_cast<std::size_t>(layer) * value_heads + h) * D + k0) * D + v);
+  f32x4 S[kQuarters][4];
 #pragma unroll
-  for (unsigned j = 0; j < kPieces; ++j) S[j] = state[tid + j * kRestoreThreads];
+  for (unsigned j = 0; j < kQuarters; ++j) {
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i) S[j][i] = state[(j * kRows + i) * (D / 4)];
+  }
   const float* key_log = key_logs + static_cast<std::size_t>(layer) * max_logged * key_elements + kh * D;
   const float* delta_log = delta_logs + static_cast<std::size_t>(layer) * max_logged * value_elements + h * D;
   for (unsigned e = tid; e < accepted * D; e += kRestoreThreads) {
@@ -1278,20 +1286,22 @@ __global__ __launch_bounds__(kRestoreThreads) void gdn_restore_recurrent_kernel(
   }
   __syncthreads();
 #pragma unroll
-  for (unsigned j = 0; j < kPieces; ++j) {
-    const unsigned piece = tid + j * kRestoreThreads;
-    const unsigned k = piece / (D / 4), v = (piece % (D / 4)) * 4;
-    f32x4 x = S[j];
+  for (unsigned j = 0; j < kQuarters; ++j) {
     for (uint32_t t = 0; t < accepted; ++t) {
-      const float decay = decays[t], key = keys[t][k];
+      const float decay = decays[t];
       const f32x4 delta = *reinterpret_cast<const f32x4*>(&deltas[t][v]);
+      const f32x4 key = *reinterpret_cast<const f32x4*>(&keys[t][j * kRows + k0]);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        x[q] = x[q] * decay;
-        x[q] = fmaf(key, delta[q], x[q]);
+      for (unsigned i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          S[j][i][q] = S[j][i][q] * decay;
+          S[j][i][q] = fmaf(key[i], delta[q], S[j][i][q]);
+        }
       }
     }
-    state[piece] = x;
+#pragma unroll
+    for (unsigned i = 0; i < 4; ++i) state[(j * kRows + i) * (D / 4)] = S[j][i];
   }
 }
 
