@@ -1248,8 +1248,15 @@ __global__ __launch_bounds__(256) void gdn_restore_conv_kernel(
 // a row, four times over: a token costs it one read each of the deltas, the decay and the
 // keys per four pieces (reads per piece made the LDS the bound), and the four quarters of
 // the state, one after the other, overlap their stores with the next one's arithmetic.
+// Streamed: the states are stored past the caches.  States of all layers that do not stay
+// in the last-level cache until they are next read come from HBM again either way, and
+// their stores then cost the loads of the same launch less (48 layers x 48 heads, three
+// sets in turn, 19 tokens: 93 -> 76 us, one token 67 -> 53 us; x 32 heads, 100 MB, 61 -> 51);
+// at 50 MB and one token, where they do stay, the plain stores win (18.1 against 19.2 us).
 constexpr unsigned kRestoreThreads = 256;
+constexpr std::size_t kRestoreStreamed = std::size_t{64} << 20;
 
+template <bool Streamed>
 __global__ __launch_bounds__(kRestoreThreads) void gdn_restore_recurrent_kernel(
     float* __restrict__ states, const float* __restrict__ key_logs, const float* __restrict__ delta_logs,
     const float* __restrict__ decay_logs, uint32_t max_logged, uint32_t accepted, uint32_t key_heads,
@@ -1301,7 +1308,14 @@ __global__ __launch_bounds__(kRestoreThreads) void gdn_restore_recurrent_kernel(
       }
     }
 #pragma unroll
-    for (unsigned i = 0; i < 4; ++i) state[(j * kRows + i) * (D / 4)] = S[j][i];
+    for (unsigned i = 0; i < 4; ++i) {
+      f32x4* to = &state[(j * kRows + i) * (D / 4)];
+      if constexpr (Streamed) {
+        __builtin_nontemporal_store(S[j][i], to);
+      } else {
+        *to = S[j][i];
+      }
+    }
   }
 }
 
@@ -2040,9 +2054,10 @@ extern "C" int32_t gfxinfer_launch_gdn_restore_prefix_all(
   if (const int32_t s = launch_status("all-layer GDN convolution prefix restore launch failed"); s != GFXI_OK) {
     return s;
   }
-  hipLaunchKernelGGL(gdn_restore_recurrent_kernel, dim3(layer_count * value_heads), dim3(kRestoreThreads), 0,
-                     st, recurrent_states, key_logs, delta_logs, decay_logs, maximum_logged_tokens,
-                     accepted_tokens, key_heads, value_heads);
+  const bool streamed = std::size_t{layer_count} * value_heads * kGdnD * kGdnD * 4 > kRestoreStreamed;
+  hipLaunchKernelGGL(streamed ? gdn_restore_recurrent_kernel<true> : gdn_restore_recurrent_kernel<false>,
+                     dim3(layer_count * value_heads), dim3(kRestoreThreads), 0, st, recurrent_states, key_logs,
+                     delta_logs, decay_logs, maximum_logged_tokens, accepted_tokens, key_heads, value_heads);
   return launch_status("all-layer GDN recurrent prefix restore launch failed");
 }
 
