@@ -10,6 +10,7 @@ using i32x4 = int __attribute__((ext_vector_type(4)));
 using u32x4 = unsigned __attribute__((ext_vector_type(4)));
 using u32x3 = unsigned __attribute__((ext_vector_type(3)));
 using u32x2 = unsigned __attribute__((ext_vector_type(2)));
+using f32x16 = float __attribute__((ext_vector_type(16)));
 
 // Buffer descriptors: one SGPR resource per stream, a lane-constant VGPR offset
 // and a wave-uniform SGPR offset per access, so a load costs no address VGPRs.

@@ -723,6 +723,12 @@ __global__ __launch_bounds__(kDirectMaxWaves * 64) void lowbit_gemm_direct_kerne
       1.0F / static_cast<float>((Format == GFXI_W4G128 ? 16 : 32) * (ABits == 4 ? 16 : 1));
   constexpr int kShift = (Format == GFXI_W4G128 ? 4 : 5) + (ABits == 4 ? 4 : 0);
   constexpr unsigned kOut = 0x80000000u;              // voffset that reads zeros
+  // Several row tiles, one token window: the scale products ws * as of a group come from
+  // the matrix core, one v_mfma_f32_16x16x1_4b_f32 (an outer product of four tiles' rows
+  // with 16 tokens) per token block instead of four conversions, two lane broadcasts and
+  // four multiplications per tile and block.  One product per output, and exact: two fp16
+  // scales have 22 significant bits between them.
+  constexpr bool kOuter = GP == 1 && R >= 2 && !Partials;
 
   extern __shared__ __align__(16) uint8_t lds_all[];
   const unsigned lane = threadIdx.x & 63u;
@@ -801,7 +807,16 @@ __global__ __launch_bounds__(kDirectMaxWaves * 64) void lowbit_gemm_direct_kerne
     // every lane of row kb by a DPP row broadcast of lane ci (no lane loads a scale that
     // another lane of its row also loads).
     u32x2 wsrow[R];
-    if constexpr (GP == 1 && !Partials) {
+    // kOuter: lane 16 kb + n holds row n of tile kb instead, one load per group.
+    unsigned short wslane[CH];
+    if constexpr (kOuter) {
+      static_assert(R <= 4, "one tile per 16 lanes");
+      const unsigned wsv = kb < valid ? (kb * groups * 16u + n) * 2u : kOut;
+#pragma unroll
+      for (unsigned ci = 0; ci < CH; ++ci) {
+        wslane[ci] = __builtin_amdgcn_raw_buffer_load_b16(weight_scales, wsv, min(g0 + ci, span.end - 1u) * 32u, 0);
+      }
+    } else if constexpr (GP == 1 && !Partials) {
       static_assert(CHG <= 16, "one scale per lane of a 16-lane row");
       const unsigned wsv = n < CHG && g0 + n < span.end ? n * 32u + kb * 8u : kOut;
 #pragma unroll
@@ -963,6 +978,14 @@ __global__ __launch_bounds__(kDirectMaxWaves * 64) void lowbit_gemm_direct_kerne
 #pragma unroll
         for (int t = 0; t < NTB; ++t) as[t] = __half2float(__ushort_as_half(asreg[ci][t])) * kInvF;
       }
+      // kOuter: block r of scale[t] holds the products of tile r's row scales and the
+      // tokens' scales.
+      f32x16 scale[NTB];
+      if constexpr (kOuter) {
+        const float ws = __half2float(__ushort_as_half(wslane[ci]));
+#pragma unroll
+        for (int t = 0; t < NTB; ++t) scale[t] = __builtin_amdgcn_mfma_f32_16x16x1f32(ws, as[t], f32x16{}, 0, 0, 0);
+      }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         if (static_cast<unsigned>(r) >= valid) break;  // wave-uniform: short last block
@@ -999,6 +1022,15 @@ __global__ __launch_bounds__(kDirectMaxWaves * 64) void lowbit_gemm_direct_kerne
                   static_cast<std::size_t>(token) * rows + (tile0 + r) * 16u + 4u * kb;
 #pragma unroll
               for (int i = 0; i < 4; ++i) args.partials[(row0 + i) * groups + g_c] = c[t][i] >> kShift;
+            }
+          }
+        } else if constexpr (kOuter) {
+#pragma unroll
+          for (int t = 0; t < NTB; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              float& a = acc[(r * NTB + t) * 4 + i];
+              a = fmaf(static_cast<float>(c[t][i]), scale[t][4 * r + i], a);
             }
           }
         } else {
@@ -1520,26 +1552,42 @@ void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipSt
   // Infinity Cache).  More tiles share each activation load and its expansion; shorter
   // chunks need fewer registers, so more waves stay resident.  A split of one canonical
   // range (the o and GDN out projections: 8-10 groups per split) runs one wave per
-  // workgroup and keeps one tile; otherwise, by row tiles x splits:
-  //   >= 2048 (gate/up): 3 tiles, 2-group chunks (32 tokens 25.3 -> 21.4 us);
-  //   1024..2047 (down as four splits): 3 tiles, 3-group chunks (16.0 -> 14.3 us);
-  //   < 1024 (q/k/v, GDN in-projection): 2 tiles, 2-group chunks at 17-32 tokens
-  //   (15.3 -> 12.2 us), 2 tiles of 5-group chunks at 9-16 tokens.
-  uint64_t tile_splits = 0;
-  for (unsigned i = 0; i < 4; ++i) {
-    const bool used = i == 0 || base_args.tile_begin[i] != base_args.tile_begin[4];
-    if (used) tile_splits += static_cast<uint64_t>(base_args.matrix[i].tiles) * base_args.splits;
-  }
+  // workgroup and keeps one tile.  Grids below 1024 row tiles x splits take 2 tiles (2-group
+  // chunks at 17-32 tokens, 5-group chunks at 9-16; 3 tiles are slower at a short K, 8.8
+  // against 7.3 us for 880 row tiles x 18 groups).  Larger ones take the R of 2, 3, 4 whose
+  // fullest CU has the fewest row tiles, R ceil(workgroups / CUs): about all workgroups of
+  // such a grid are resident at once, so the launch lasts as long as that CU (W4 x 32
+  // tokens, 3 against 4 tiles: 1280 row tiles 14.9 / 16.9 us, 1728 row tiles 20.5 / 17.9,
+  // 4096 row tiles 40.5 / 37.9); within a thirtieth of each other the larger R (9496 row
+  // tiles 89.3 / 86.6).  Chunks are 2 groups; with 3 tiles 3 groups where a range has no
+  // more than nine (8.5 groups, W3 down projection: 13.4 against 14.7 us; 10 groups, 1030
+  // row tiles: 15.9 against 14.3).
+  const auto blocks_of = [&](unsigned r) {
+    uint64_t blocks = 0;
+    for (unsigned i = 0; i < 4; ++i) {
+      const bool used = i == 0 || base_args.tile_begin[i] != base_args.tile_begin[4];
+      if (used) blocks += (static_cast<uint64_t>(base_args.matrix[i].tiles) + r - 1) / r;
+    }
+    return blocks * base_args.splits;
+  };
   const bool one_range = min_range_count(base_args.groups, base_args.splits) <= 1;
-  int shape;  // 1: 1 x 4, 2: 2 x 5, 3: 3 x 2, 4: 3 x 3, 5: 2 x 2
+  int shape;  // R x CH -- 1: 1 x 4, 2: 2 x 5, 3: 3 x 2, 4: 3 x 3, 5: 2 x 2, 6: 4 x 2
   if (one_range) {
     shape = 1;
-  } else if (tile_splits >= 2048) {
-    shape = 3;
-  } else if (tile_splits >= 1024) {
-    shape = 4;
-  } else {
+  } else if (blocks_of(1) < 4 * kComputeUnits) {
     shape = batch > 16 ? 5 : 2;
+  } else {
+    unsigned best = 2;
+    uint64_t fullest = 2 * ((blocks_of(2) + kComputeUnits - 1) / kComputeUnits);
+    for (unsigned r = 3; r <= 4; ++r) {
+      const uint64_t tiles = r * ((blocks_of(r) + kComputeUnits - 1) / kComputeUnits);
+      if (tiles * 30 <= fullest * 31) {
+        best = r;
+        fullest = tiles;
+      }
+    }
+    const unsigned split = base_args.groups / base_args.splits;
+    shape = best == 2 ? 5 : (best == 4 ? 6 : (split <= 9 * range_count(split) ? 4 : 3));
   }
   (void)total_tiles;
   if (batch <= 4) {
@@ -1551,6 +1599,8 @@ void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipSt
       case 2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 5, 2, HalfOut, Partials>, 2, 1); break;
       case 3: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 3, HalfOut, Partials>, 3, 1); break;
       case 4: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 3, 3, HalfOut, Partials>, 3, 1); break;
+      case 5: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 2, HalfOut, Partials>, 2, 1); break;
+      case 6: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 4, HalfOut, Partials>, 4, 1); break;
       default: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 4, 1, HalfOut, Partials>, 1, 1); break;
     }
   } else if constexpr (ABits == 8) {
@@ -1561,6 +1611,7 @@ void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipSt
       case 3: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 3, HalfOut, Partials>, 3, 2); break;
       case 4: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 3, 3, HalfOut, Partials>, 3, 2); break;
       case 5: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 2, HalfOut, Partials>, 2, 2); break;
+      case 6: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 4, HalfOut, Partials>, 4, 2); break;
       default: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 4, 1, HalfOut, Partials>, 1, 2); break;
     }
   }

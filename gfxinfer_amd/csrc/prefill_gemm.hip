@@ -30,7 +30,6 @@ namespace {
 
 using i32x8 = int __attribute__((ext_vector_type(8)));
 using f32x4 = float __attribute__((ext_vector_type(4)));
-using f32x16 = float __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------------------
 // FP6 operands.  A lane's 32 columns are four dwords of eight nibbles (column 8 j + i in
