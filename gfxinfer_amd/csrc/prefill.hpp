@@ -60,6 +60,26 @@ struct GdnPrefillPass {
 };
 int32_t gdn_prefill(const GdnPrefillPass& pass, hipStream_t stream);
 
+// gfxinfer_launch_gated_attention_decode_block_quantize_i4 over any number of tokens: token
+// t at position + t, each 32-token block with the splits and the arithmetic of a launch of
+// its own.  The workspace holds at least one block's partial results
+// (gfxinfer_attention_workspace_bytes(32, ..., position + tokens)).
+struct PrefillAttention {
+  const uint16_t* query;        // [tokens][q_heads * head_size]
+  const float* gate;            // [tokens][q_heads][2 * head_size]
+  const uint16_t* key_cache;
+  const uint16_t* value_cache;
+  uint16_t* output;             // [tokens][q_heads * head_size]
+  uint8_t* codes;
+  uint16_t* scales;
+  uint64_t position;
+  std::size_t capacity;
+  uint32_t tokens, q_heads, kv_heads, head_size;
+  float* workspace;
+  std::size_t workspace_bytes;
+};
+int32_t prefill_attention(const PrefillAttention& attention, hipStream_t stream);
+
 // The block launchers' kernels over any number of rows.
 int32_t quantize_activation_rows(const uint16_t* input, uint8_t* codes, uint16_t* scales, std::size_t columns,
                                  uint32_t rows, hipStream_t stream);

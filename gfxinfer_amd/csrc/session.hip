@@ -546,9 +546,8 @@ struct gfxinfer_session {
   // ---- wide prefill pass --------------------------------------------------------
   // The layer block over T > 32 tokens: the block kernels' arithmetic value for value (the
   // GEMM in prefill_gemm.hip and the GDN pass in qwen_ops.hip; the others are the block
-  // launchers' kernels over more rows, or, for the attention, its launches one 32-token
-  // block after the other), so every state, cache and hidden row equals the block-by-block
-  // pass.
+  // launchers' kernels over more rows or blocks), so every state, cache and hidden row
+  // equals the block-by-block pass.
 
   // A4 codes and scales in wide_codes / wide_scales -> the GEMM's operand.
   int32_t wide_operand(std::size_t columns, unsigned T, PrefillOperand& out) {
@@ -597,14 +596,16 @@ struct gfxinfer_session {
       GFXI_TRY(wide_gemm({{&L.q, wide_main}, {&L.k, wide_k}, {&L.v, wide_v}}, in, T));
       const std::size_t offset = L.state_index * config.maximum_context_tokens * kv_rows;
       GFXI_TRY(wide_rope_append(L, key_caches + offset, value_caches + offset, current_position, T));
-      for (unsigned a = 0; a < T; a += kMaxBlock) {
-        GFXI_TRY(gfxinfer_launch_gated_attention_decode_block_quantize_i4(
-            wide_query + a * attn_width, wide_main + a * q_rows, key_caches + offset, value_caches + offset,
-            wide_attention + a * attn_width, wide_codes + a * attn_width / 2, wide_scales + a * (attn_width / kGroup),
-            current_position + a + 1, config.maximum_context_tokens, std::min(kMaxBlock, T - a),
-            spec.attention_head_count, spec.kv_head_count, spec.attention_head_size, attention_workspace,
-            attention_workspace_bytes, stream));
-      }
+      // The partial results go where the MLP's gate and up rows come later, or to the block
+      // pass's workspace when a long context makes that the larger one.
+      const std::size_t mlp_bytes = 2 * wide_tokens * I * 4;
+      const bool in_mlp = mlp_bytes > attention_workspace_bytes;
+      GFXI_TRY(prefill_attention({wide_query, wide_main, key_caches + offset, value_caches + offset, wide_attention,
+                                  wide_codes, wide_scales, current_position, config.maximum_context_tokens, T,
+                                  spec.attention_head_count, spec.kv_head_count, spec.attention_head_size,
+                                  in_mlp ? wide_gate : attention_workspace,
+                                  in_mlp ? mlp_bytes : attention_workspace_bytes},
+                                 stream));
     } else {
       GFXI_TRY(wide_gemm({{&L.qkv, wide_main}, {&L.z, wide_z}, {&L.a, wide_a}, {&L.b, wide_b}}, in, T));
       // As one window: from the states into the snapshot buffers, swapped after the pass.
