@@ -176,6 +176,7 @@ SIGNATURES: dict[str, tuple] = {
     "gfxinfer_session_set_layer_trace": (I32, [P, P, SZ]),
     "gfxinfer_session_layer_trace_bytes": (SZ, [P]),
     "gfxinfer_session_prefill": (I32, [P, P, SZ, I32, P]),
+    "gfxinfer_debug_model_wide_scratch": (SZ, [P, I32]),
     "gfxinfer_session_generate": (I32, [P, P, SZ, P, P, P, P]),
     "gfxinfer_depth_policy_create": (I32, [U32, P]),
     "gfxinfer_depth_policy_destroy": (None, [P]),

@@ -392,6 +392,7 @@ namespace {
 void free_model(gfxinfer_model* model) {
   (void)hipSetDevice(model->device);
   if (model->stream != nullptr) (void)hipStreamSynchronize(model->stream);
+  if (model->wide.data != nullptr) (void)hipFree(model->wide.data);
   if (model->arena != nullptr) (void)hipFree(model->arena);
   if (model->stream != nullptr) (void)hipStreamDestroy(model->stream);
   delete model;
@@ -412,6 +413,16 @@ void release_model_reference(gfxinfer_model* model) {
   }
   if (last) free_model(model);
 }
+
+bool release_wide_scratch(gfxinfer_model* model) {
+  const std::lock_guard<std::mutex> hold(model->wide.use);
+  if (model->wide.data == nullptr || hipSetDevice(model->device) != hipSuccess) return false;
+  (void)hipStreamSynchronize(model->stream);
+  (void)hipFree(model->wide.data);
+  model->wide.data = nullptr;
+  model->wide.bytes = 0;
+  return true;
+}
 }  // namespace gfx950
 
 extern "C" void gfxinfer_model_destroy(gfxinfer_model* model) {
@@ -423,6 +434,14 @@ extern "C" void gfxinfer_model_destroy(gfxinfer_model* model) {
     unused = model->sessions == 0;
   }
   if (unused) gfx950::free_model(model);
+}
+
+extern "C" size_t gfxinfer_debug_model_wide_scratch(gfxinfer_model* model, int32_t refuse) {
+  if (model == nullptr) return 0;
+  if (refuse > 0) (void)gfx950::release_wide_scratch(model);
+  const std::lock_guard<std::mutex> hold(model->wide.use);
+  if (refuse >= 0) model->wide.refused = refuse > 0;
+  return model->wide.bytes;
 }
 
 extern "C" size_t gfxinfer_model_spec_tensor_count(const gfxinfer_model_spec* spec) {

@@ -15,6 +15,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -193,9 +194,8 @@ struct gfxinfer_session {
   uint16_t *key_caches{}, *value_caches{}, *mtp_key_cache{}, *mtp_value_cache{};
   uint32_t* host_result{nullptr};  // pinned
 
-  // Wide prefill: passes of up to wide_tokens prompt tokens over every layer (0: none, the
-  // context is one block or the buffers did not fit).
-  std::size_t wide_tokens{0};
+  // Buffers of a wide prefill pass: places in the model's scratch, set by each pass
+  // (wide_buffers) for its own duration.
   uint16_t *wide_hidden_a{}, *wide_hidden_b{}, *wide_post{}, *wide_conditioning{}, *wide_concat{};
   uint16_t *wide_mtp_input{}, *wide_query{}, *wide_key{}, *wide_attention{};
   uint8_t *wide_codes{}, *wide_fragments{};
@@ -203,7 +203,8 @@ struct gfxinfer_session {
   float2* wide_meta{};
   float *wide_main{}, *wide_z{}, *wide_a{}, *wide_b{}, *wide_k{}, *wide_v{}, *wide_mixed{};
   float *wide_convolved{}, *wide_gates{};
-  float *wide_update{}, *wide_gate{}, *wide_up{};
+  float *wide_update{}, *wide_gate{}, *wide_up{}, *wide_partials{};
+  std::size_t wide_partials_bytes{0};
 
   std::array<Graph, 2> graphs{};
 
@@ -549,6 +550,88 @@ struct gfxinfer_session {
   // launchers' kernels over more rows or blocks), so every state, cache and hidden row
   // equals the block-by-block pass.
 
+  // Lays the pass's buffers out from `base` and returns their bytes (base null: the size
+  // alone).  Rows of kWideTokens tokens, whatever the pass or the context.  The steps of a
+  // layer share one region: the attention layer's main .. attention and the GDN layer's
+  // main .. gates (its main is the attention layer's) are dead when gate and up are written,
+  // and the attention's partial results take what lies between its own buffers and the end
+  // of update, which holds nothing during the mixer.  The MTP rows follow the last layer.
+  std::size_t wide_buffers(uint8_t* base) {
+    constexpr std::size_t W = kWideTokens;
+    static_assert(W % kMaxBlock == 0, "whole blocks and whole 16-token tiles");
+    std::size_t cursor = 0;
+    const auto take = [&](auto*& slot, std::size_t bytes) {
+      slot = base == nullptr ? nullptr : reinterpret_cast<std::remove_reference_t<decltype(slot)>>(base + cursor);
+      cursor = align256(cursor + bytes);
+    };
+    const std::size_t max_k = std::max({I, 2 * H, attn_width, gdn_value});
+    const std::size_t planes = std::max({gfxinfer_gemm_split_count(H, I, 1), gfxinfer_gemm_split_count(H, attn_width, 1),
+                                         gfxinfer_gemm_split_count(H, gdn_value, 1)});
+    take(wide_hidden_a, W * H * 2);
+    take(wide_hidden_b, W * H * 2);
+    take(wide_post, W * H * 2);
+    take(wide_codes, W * max_k / 2);
+    take(wide_scales, W * (max_k / kGroup) * 2);
+    take(wide_fragments, prefill_fragment_bytes(max_k, W));
+    take(wide_meta, prefill_meta_bytes(max_k, W));
+    const std::size_t layer = cursor;
+    take(wide_gate, W * I * 4);
+    take(wide_up, W * I * 4);
+    const std::size_t mlp_end = cursor;
+    cursor = layer;
+    take(wide_main, W * std::max(q_rows, channels) * 4);
+    take(wide_k, W * kv_rows * 4);
+    take(wide_v, W * kv_rows * 4);
+    take(wide_query, W * attn_width * 2);
+    take(wide_key, W * kv_rows * 2);
+    take(wide_attention, W * attn_width * 2);
+    const std::size_t partials = cursor;
+    take(wide_z, W * gdn_value * 4);
+    take(wide_a, W * spec.gdn_value_head_count * 4);
+    take(wide_b, W * spec.gdn_value_head_count * 4);
+    take(wide_mixed, W * gdn_value * 4);
+    take(wide_convolved, W * channels * 4);
+    take(wide_gates, 2 * W * spec.gdn_value_head_count * 4);
+    cursor = std::max(cursor, mlp_end);
+    const std::size_t update = cursor;
+    take(wide_conditioning, W * H * 2);
+    take(wide_concat, W * 2 * H * 2);
+    take(wide_mtp_input, W * H * 2);
+    const std::size_t mtp_end = cursor;
+    cursor = update;
+    take(wide_update, planes * W * H * 4);
+    cursor = std::max(cursor, mtp_end);
+    wide_partials = base == nullptr ? nullptr : reinterpret_cast<float*>(base + partials);
+    wide_partials_bytes = cursor - partials;
+    return cursor;
+  }
+
+  // The model's scratch for a wide pass, allocated at the first one (wide.use held).  False:
+  // it cannot be had, or would take more than half of the memory still free, which is left
+  // to the sessions and the program; the prompt then runs in blocks.
+  bool wide_scratch() {
+    WideScratch& wide = model->wide;
+    const std::size_t bytes = wide_buffers(nullptr);
+    if (wide.data == nullptr) {
+      // A capture elsewhere in the program does not meet this allocation.
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+      std::size_t free_bytes = 0, total_bytes = 0;
+      if (wide.refused || (hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && free_bytes / 2 >= bytes)) {
+        void* data = nullptr;
+        if (hipMalloc(&data, wide.refused ? std::size_t{1} << 50 : bytes) == hipSuccess) {
+          wide.data = static_cast<uint8_t*>(data);
+          wide.bytes = bytes;
+        }
+      }
+      (void)hipGetLastError();  // a refused allocation is no error of the launches that follow
+      if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (wide.data == nullptr) return false;
+    }
+    wide_buffers(wide.data);
+    return true;
+  }
+
   // A4 codes and scales in wide_codes / wide_scales -> the GEMM's operand.
   int32_t wide_operand(std::size_t columns, unsigned T, PrefillOperand& out) {
     out = {wide_fragments, wide_meta, (T + 15) / 16};
@@ -596,15 +679,14 @@ struct gfxinfer_session {
       GFXI_TRY(wide_gemm({{&L.q, wide_main}, {&L.k, wide_k}, {&L.v, wide_v}}, in, T));
       const std::size_t offset = L.state_index * config.maximum_context_tokens * kv_rows;
       GFXI_TRY(wide_rope_append(L, key_caches + offset, value_caches + offset, current_position, T));
-      // The partial results go where the MLP's gate and up rows come later, or to the block
-      // pass's workspace when a long context makes that the larger one.
-      const std::size_t mlp_bytes = 2 * wide_tokens * I * 4;
-      const bool in_mlp = mlp_bytes > attention_workspace_bytes;
+      // The partial results go to the free part of the layer's region, or to the block pass's
+      // workspace when a long context makes that the larger one.
+      const bool in_scratch = wide_partials_bytes > attention_workspace_bytes;
       GFXI_TRY(prefill_attention({wide_query, wide_main, key_caches + offset, value_caches + offset, wide_attention,
                                   wide_codes, wide_scales, current_position, config.maximum_context_tokens, T,
                                   spec.attention_head_count, spec.kv_head_count, spec.attention_head_size,
-                                  in_mlp ? wide_gate : attention_workspace,
-                                  in_mlp ? mlp_bytes : attention_workspace_bytes},
+                                  in_scratch ? wide_partials : attention_workspace,
+                                  in_scratch ? wide_partials_bytes : attention_workspace_bytes},
                                  stream));
     } else {
       GFXI_TRY(wide_gemm({{&L.qkv, wide_main}, {&L.z, wide_z}, {&L.a, wide_a}, {&L.b, wide_b}}, in, T));
@@ -654,8 +736,13 @@ struct gfxinfer_session {
 
   // T > kMaxBlock prompt tokens in one pass, as blocks of 32 would leave the session: states,
   // caches, MTP cache, positions, and the last block's hidden rows (and, with `head`, its
-  // logits and greedy tokens, the last of which goes to *next).
-  int32_t wide_pass(const uint32_t* tokens, unsigned T, bool sync_mtp, bool head, uint32_t* next) {
+  // logits and greedy tokens, the last of which goes to *next).  *ran = false: there is no
+  // scratch for it, and nothing has run.
+  int32_t wide_pass(const uint32_t* tokens, unsigned T, bool sync_mtp, bool head, uint32_t* next, bool* ran) {
+    // The model's sessions share the scratch and the stream: passes follow one another.
+    const std::lock_guard<std::mutex> hold(model->wide.use);
+    *ran = wide_scratch();
+    if (!*ran) return ok();
     const bool previous = current_position != 0;  // a hidden state for the position before
     const auto copy = [&](void* to, const void* from, std::size_t bytes) -> int32_t {
       if (auto e = hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, stream); e != hipSuccess) {
@@ -663,7 +750,6 @@ struct gfxinfer_session {
       }
       return ok();
     };
-    if (sync_mtp && previous) GFXI_TRY(copy(wide_conditioning, last_hidden, H * 2));
     GFXI_TRY(wide_gather(wide_hidden_a, tokens, T));
     GFXI_TRY(gfxinfer_launch_rms_norm_quantize_i4(wide_hidden_a, layers.front().input_norm, nullptr, wide_codes,
                                                   wide_scales, H, T, spec.rms_norm_epsilon, 1, stream));
@@ -672,6 +758,7 @@ struct gfxinfer_session {
       GFXI_TRY(wide_layer(layers[i], current, other, T, i + 1 < layers.size() ? layers[i + 1].input_norm : final_norm));
       std::swap(current, other);
     }
+    if (sync_mtp && previous) GFXI_TRY(copy(wide_conditioning, last_hidden, H * 2));  // before hidden_a's rows go
     // The last block's rows (the rows after them keep the block before, as its pass left them).
     const unsigned last = (T - 1) % kMaxBlock + 1, first = T - last;
     if (last < kMaxBlock) {
@@ -702,7 +789,7 @@ struct gfxinfer_session {
     return ok();
   }
 
-  // Chunked prefill: the target over the prompt in passes of up to kMaxBlock or wide_tokens
+  // Chunked prefill: the target over the prompt in passes of up to kMaxBlock or kWideTokens
   // tokens and, with sync_mtp, the MTP cache over the same positions (entry j from token
   // j + 1 and the target hidden state of position j), the state the serial loop of
   // cli/main.cpp:1055-1069 (greedy_step(p0); then mtp_draft(p_i) and greedy_step(p_i))
@@ -721,11 +808,12 @@ struct gfxinfer_session {
     while (valid < count && tokens[valid] < spec.vocabulary_size) ++valid;
     if (valid < count) valid -= valid % kMaxBlock;
     uint32_t outputs[kMaxBlock];
+    bool wide = layer_trace == nullptr;
     for (std::size_t a = 0, step = 0; a < count; a += step) {
-      step = std::min(wide_tokens, valid > a ? valid - a : 0);
-      if (step >= kWideMinimum && layer_trace == nullptr) {
-        GFXI_TRY(wide_pass(tokens + a, static_cast<unsigned>(step), sync_mtp, a + step == valid, next));
-        continue;
+      step = std::min(kWideTokens, valid > a ? valid - a : 0);
+      if (wide && step >= kWideMinimum) {
+        GFXI_TRY(wide_pass(tokens + a, static_cast<unsigned>(step), sync_mtp, a + step == valid, next, &wide));
+        if (wide) continue;
       }
       step = std::min<std::size_t>(kMaxBlock, count - a);
       const auto T = static_cast<unsigned>(step);
@@ -1066,9 +1154,8 @@ void bind_mlp(const gfxinfer_model& m, const std::string& p, Layer& L, bool& mis
 
 }  // namespace
 
-extern "C" int32_t gfxinfer_session_create(gfxinfer_model* model,
-                                           const gfxinfer_session_config* config,
-                                           gfxinfer_session** out) {
+namespace {
+int32_t create_session(gfxinfer_model* model, const gfxinfer_session_config* config, gfxinfer_session** out) {
   return guarded([&]() -> int32_t {
     if (model == nullptr || config == nullptr || out == nullptr ||
         config->maximum_context_tokens == 0 ||
@@ -1216,64 +1303,18 @@ extern "C" int32_t gfxinfer_session_create(gfxinfer_model* model,
         {"mtp_key_cache", reinterpret_cast<void**>(&s->mtp_key_cache), mtp_kv_bytes},
         {"mtp_value_cache", reinterpret_cast<void**>(&s->mtp_value_cache), mtp_kv_bytes},
     };
+    std::size_t cursor = 0;
     std::vector<std::size_t> offsets;
-    const auto lay_out = [&]() {
-      std::size_t cursor = 0;
-      offsets.clear();
-      for (const auto& b : s->buffers) {
-        cursor = align256(cursor);
-        offsets.push_back(cursor);
-        cursor += b.bytes;
-      }
-      s->arena_bytes = align256(cursor);
-    };
-    const std::size_t block_buffers = s->buffers.size();
-    if (ctx >= kWideMinimum) {
-      s->wide_tokens = std::min(kWideTokens, ctx);
-      const std::size_t W = (s->wide_tokens + 15) / 16 * 16;
-      const std::size_t update_planes = std::max({gfxinfer_gemm_split_count(s->H, s->I, 1),
-                                                  gfxinfer_gemm_split_count(s->H, s->attn_width, 1),
-                                                  gfxinfer_gemm_split_count(s->H, s->gdn_value, 1)});
-      s->buffers.insert(s->buffers.end(), {
-          {"wide_hidden_a", reinterpret_cast<void**>(&s->wide_hidden_a), W * s->H * 2},
-          {"wide_hidden_b", reinterpret_cast<void**>(&s->wide_hidden_b), W * s->H * 2},
-          {"wide_post", reinterpret_cast<void**>(&s->wide_post), W * s->H * 2},
-          {"wide_conditioning", reinterpret_cast<void**>(&s->wide_conditioning), W * s->H * 2},
-          {"wide_concat", reinterpret_cast<void**>(&s->wide_concat), W * 2 * s->H * 2},
-          {"wide_mtp_input", reinterpret_cast<void**>(&s->wide_mtp_input), W * s->H * 2},
-          {"wide_query", reinterpret_cast<void**>(&s->wide_query), W * s->attn_width * 2},
-          {"wide_key", reinterpret_cast<void**>(&s->wide_key), W * s->kv_rows * 2},
-          {"wide_attention", reinterpret_cast<void**>(&s->wide_attention), W * s->attn_width * 2},
-          {"wide_codes", reinterpret_cast<void**>(&s->wide_codes), W * max_k / 2},
-          {"wide_scales", reinterpret_cast<void**>(&s->wide_scales), W * (max_k / 128) * 2},
-          {"wide_fragments", reinterpret_cast<void**>(&s->wide_fragments), prefill_fragment_bytes(max_k, W)},
-          {"wide_meta", reinterpret_cast<void**>(&s->wide_meta), prefill_meta_bytes(max_k, W)},
-          {"wide_main", reinterpret_cast<void**>(&s->wide_main), W * std::max(s->q_rows, s->channels) * 4},
-          {"wide_z", reinterpret_cast<void**>(&s->wide_z), W * s->gdn_value * 4},
-          {"wide_a", reinterpret_cast<void**>(&s->wide_a), W * sp.gdn_value_head_count * 4},
-          {"wide_b", reinterpret_cast<void**>(&s->wide_b), W * sp.gdn_value_head_count * 4},
-          {"wide_k", reinterpret_cast<void**>(&s->wide_k), W * s->kv_rows * 4},
-          {"wide_v", reinterpret_cast<void**>(&s->wide_v), W * s->kv_rows * 4},
-          {"wide_mixed", reinterpret_cast<void**>(&s->wide_mixed), W * s->gdn_value * 4},
-          {"wide_convolved", reinterpret_cast<void**>(&s->wide_convolved), W * s->channels * 4},
-          {"wide_gates", reinterpret_cast<void**>(&s->wide_gates), 2 * W * sp.gdn_value_head_count * 4},
-          {"wide_update", reinterpret_cast<void**>(&s->wide_update), update_planes * W * s->H * 4},
-          {"wide_gate", reinterpret_cast<void**>(&s->wide_gate), W * s->I * 4},
-          {"wide_up", reinterpret_cast<void**>(&s->wide_up), W * s->I * 4},
-      });
+    for (const auto& b : s->buffers) {
+      cursor = align256(cursor);
+      offsets.push_back(cursor);
+      cursor += b.bytes;
     }
-    lay_out();
+    s->arena_bytes = align256(cursor);
     std::size_t free_bytes = 0, total_bytes = 0;
     int32_t status = ok();
-    const hipError_t memory_info = hipMemGetInfo(&free_bytes, &total_bytes);
-    if (memory_info == hipSuccess && s->arena_bytes > free_bytes && s->wide_tokens != 0) {
-      // Without the wide pass's buffers the session may still fit: prompts then run in blocks.
-      s->buffers.resize(block_buffers);
-      s->wide_tokens = 0;
-      lay_out();
-    }
-    if (memory_info != hipSuccess) {
-      status = hip_fail(memory_info, "hipMemGetInfo before session allocation failed");
+    if (auto e = hipMemGetInfo(&free_bytes, &total_bytes); e != hipSuccess) {
+      status = hip_fail(e, "hipMemGetInfo before session allocation failed");
     } else if (s->arena_bytes > free_bytes) {
       status = fail(GFXI_OUT_OF_MEMORY, "decode session arena exceeds currently free GPU memory");
     } else if (auto e2 = hipMalloc(reinterpret_cast<void**>(&s->arena), s->arena_bytes);
@@ -1313,6 +1354,19 @@ extern "C" int32_t gfxinfer_session_create(gfxinfer_model* model,
     *out = s;
     return ok();
   });
+}
+}  // namespace
+
+extern "C" int32_t gfxinfer_session_create(gfxinfer_model* model,
+                                           const gfxinfer_session_config* config,
+                                           gfxinfer_session** out) {
+  const int32_t status = create_session(model, config, out);
+  // What needs memory comes before the scratch of earlier prompts.
+  if ((status == GFXI_OUT_OF_MEMORY || status == GFXI_HIP_ERROR) && release_wide_scratch(model)) {
+    (void)hipGetLastError();
+    return create_session(model, config, out);
+  }
+  return status;
 }
 
 extern "C" void gfxinfer_session_destroy(gfxinfer_session* session) { delete session; }

@@ -293,14 +293,22 @@ int32_t gfxinfer_session_set_layer_trace(gfxinfer_session* session, void* device
 /* Chunked prefill.  The reference prefills a prompt with one greedy_step per token and,
  * when MTP is on, an mtp_draft per token from the second on (cli/main.cpp:1055-1069);
  * this runs the target over the prompt in wide passes (65 to 512 tokens) and blocks of up
- * to 32 tokens and, with sync_mtp != 0, advances the MTP K/V cache over the same positions in batches (entry j
- * from token j + 1 and the target's hidden state at position j), leaving the target,
- * GDN, KV and MTP cache state and the positions as that serial loop leaves them.
+ * to 32 tokens and, with sync_mtp != 0, advances the MTP K/V cache over the same positions
+ * in batches (entry j from token j + 1 and the target's hidden state at position j),
+ * leaving the target, GDN, KV and MTP cache state and the positions as that serial loop
+ * leaves them.  The first wide pass on a model allocates its scratch (about 150 MB at the
+ * reference's widths, not in arena_bytes), which the model's sessions share; it is given
+ * back with the model, or earlier when a session creation needs the memory.  Where it
+ * cannot be had, or would take more than half of the free memory, the prompt runs in blocks.
  * *next_token = the greedy token after the last prompt token.  Requires a fresh
  * session or, with sync_mtp, an aligned one (mtp_position + 1 == position).  No
  * reference counterpart (the reference roadmap's "fast prefill", README.md:211-218). */
 int32_t gfxinfer_session_prefill(gfxinfer_session* session, const uint32_t* tokens, size_t count,
                                  int32_t sync_mtp, uint32_t* next_token);
+/* Test hook, no reference counterpart: bytes of wide-pass scratch the model holds.
+ * refuse > 0 gives it back first and makes every later allocation of it fail, 0 lets it
+ * succeed again, < 0 only asks. */
+size_t gfxinfer_debug_model_wide_scratch(gfxinfer_model* model, int32_t refuse);
 
 /* Online MTP depth selection ("Online MTP depth selection based on accepted tokens
  * per millisecond", docs/ROADMAP.md:51; not implemented by the reference).  The

@@ -129,3 +129,59 @@ def test_wide_prefill_refuses_what_blocks_refuse(model):
     _same(a, b, 32)
     a.close()
     b.close()
+
+
+def _scratch(model, refuse=-1):
+    from gfxinfer_amd import lib
+    return int(lib().gfxinfer_debug_model_wide_scratch(model.handle, refuse))
+
+
+def test_scratch_belongs_to_the_model(model):
+    """Sessions hold no memory for wide passes, the first such pass allocates the model's scratch, later sessions
+    use the same one, and a session creation that does not fit gets it back."""
+    from gfxinfer_amd import GfxinferError
+    from gfxinfer_amd.runtime import QwenDecodeSession
+    prompt = np.random.default_rng(9).integers(0, 1000, 200).astype(np.uint32)
+    _scratch(model, 1), _scratch(model, 0)
+    small, large = QwenDecodeSession(model, 64), QwenDecodeSession(model, 65)
+    assert large.summary().arena_bytes - small.summary().arena_bytes < 1 << 20
+    small.close(), large.close()
+    a, b, c = (QwenDecodeSession(model, CONTEXT, 0, keep_logits=True) for _ in range(3))
+    say("prompts on one scratch")
+    _blocks(a, prompt[:100], True)
+    b.prefill(prompt[:64])
+    assert _scratch(model) == 0                       # short prompts need none
+    c.prefill(prompt[:100])
+    held = _scratch(model)
+    assert held > 0 and c.prefill(prompt[100:]) == _blocks(a, prompt[100:], True)
+    b.prefill(prompt[64:])
+    assert _scratch(model) == held
+    _same(a, c, 4)
+    with pytest.raises(GfxinferError):
+        QwenDecodeSession(model, 1 << 40)             # exceeds any memory: refused before anything is launched
+    assert _scratch(model) == 0
+    say("prompts after the scratch was given back")
+    assert c.prefill(prompt) == _blocks(a, prompt, True) and _scratch(model) == held
+    _same(a, c, 8)
+    for s in (a, b, c):
+        s.close()
+
+
+def test_prompt_without_scratch_runs_in_blocks(model):
+    """The scratch's allocation fails: the same results, and nothing later sees the failure."""
+    from gfxinfer_amd.runtime import QwenDecodeSession
+    prompt = np.random.default_rng(10).integers(0, 1000, 600).astype(np.uint32)
+    a, b = (QwenDecodeSession(model, CONTEXT, 5, keep_logits=True) for _ in range(2))
+    want = _blocks(a, prompt, True)
+    _scratch(model, 1)
+    try:
+        say("prompt without scratch")
+        assert b.prefill(prompt) == want and _scratch(model) == 0
+    finally:
+        _scratch(model, 0)
+    _same(a, b, 24)
+    ra, rb = a.speculative_step(want, 4), b.speculative_step(want, 4)
+    assert (ra.tokens, ra.accepted_drafts) == (rb.tokens, rb.accepted_drafts)
+    _same(a, b, 5)
+    a.close()
+    b.close()
