@@ -1522,6 +1522,60 @@ unsigned choose_waves(uint32_t groups) {
   return waves;
 }
 
+// Row tiles per wave (R) and groups per load chunk (CH) of the direct kernel at 9-32 tokens,
+// by grid shape.  More tiles share each activation load and its expansion; shorter chunks
+// need fewer registers, so more waves stay resident.  Measured on MI355X with weights
+// rotated past the last-level cache; all shapes give the same bits.
+//   * A split of one canonical range (the o and GDN out projections: 8-10 groups per split)
+//     runs one wave per workgroup and keeps one tile.
+//   * Below 1024 row tiles x splits: 2 tiles, 2-group chunks at 17-32 tokens, 5-group chunks
+//     at 9-16 (W4, 880 row tiles, 40 groups: 32 tokens 12.1 us against 12.9-14.1 with 3 or 4
+//     tiles, 12 tokens 10.0 against 10.7-11.3).  From 60 groups on, unsplit, 3 or 4 tiles
+//     are faster (880 x 136 groups x 32 tokens: 38.8 against 31.6); such matrices come in
+//     split-K planes here.
+//   * Larger grids: the R whose fullest CU has the least to do.  That CU holds
+//     R ceil(workgroups / CUs) tiles, and a tile costs less the more of them share a wave:
+//     with 3 tiles 0.95 and with 4 tiles 0.90 of what it costs with 2, with 4 tiles at 17-32
+//     tokens and four to seven ranges 0.83 (W4 x 32 tokens x 40 groups, 2 / 3 / 4 tiles:
+//     1100 row tiles 16.4 / 14.8 / 16.6 us, 1728 21.1 / 21.0 / 18.3, 2560 28.3 / 26.7 / 25.7,
+//     9496 92.5 / 88.1 / 84.8; x 80 groups, eight waves that hold a CU alone: 2560 49.1 /
+//     48.9 / 49.3; 12 tokens x 40 groups: 1100 12.0 / 11.8 / 13.4, 2560 19.9 / 21.7 / 21.4,
+//     9496 69.8 / 71.0 / 68.9).  More than 2560 row tiles x 80 groups, which no model here
+//     has, can miss the best by 7 % (3300 x 32 tokens W3: 57.9 us, 54.1 with 3 tiles).
+//   * Up to three ranges a workgroup is two or three waves, several share a CU, and the
+//     launch is as long as one of them: while the fullest CU holds no more than four
+//     workgroups of 2 tiles, those (1728 row tiles, 18 groups, W3: 32 tokens 11.2 us against
+//     13.5 with 4 tiles, 12 tokens 9.0 against 10.4), in 5-group chunks where a range is two
+//     of them and no CU holds a fourth (1100 row tiles 9.8 against 10.3 us).
+//   * 3 tiles: 3-group chunks for ranges of more than eight and at most nine groups (8.5
+//     groups, W3 down projection: 13.7 against 13.9 us, at 12 tokens 10.1 against 10.7),
+//     which they cut evenly, else 2-group ones (8 groups, W4 x 2176 row tiles: 14.7 against
+//     16.8; 10 groups, 1100 row tiles: 14.8 against 16.4).
+enum DirectShape : int { k1x4 = 1, k2x5, k3x2, k3x3, k2x2, k4x2 };  // R x CH
+
+int direct_shape(const GemmArgs& args) {
+  if (min_range_count(args.groups, args.splits) <= 1) return k1x4;
+  const auto blocks_of = [&](unsigned r) {
+    uint64_t blocks = 0;
+    for (unsigned i = 0; i < 4; ++i) {
+      // unused trailing slots repeat the last matrix with zero tiles
+      const bool used = i == 0 || args.tile_begin[i] != args.tile_begin[4];
+      if (used) blocks += (static_cast<uint64_t>(args.matrix[i].tiles) + r - 1) / r;
+    }
+    return blocks * args.splits;
+  };
+  const bool two_blocks = args.batch > 16;
+  if (blocks_of(1) < 4 * kComputeUnits) return two_blocks ? k2x2 : k2x5;
+  const auto fullest = [&](unsigned r) { return r * ((blocks_of(r) + kComputeUnits - 1) / kComputeUnits); };
+  const unsigned split = args.groups / args.splits, ranges = range_count(split);
+  const uint64_t tiles2 = fullest(2);
+  if (ranges <= 3 && tiles2 <= 8) return ranges <= 2 && tiles2 <= 6 ? k2x5 : k2x2;
+  const uint64_t cost2 = tiles2 * 100, cost3 = fullest(3) * 95, cost4 = fullest(4) * (two_blocks && ranges >= 4 && ranges < 8 ? 83 : 90);
+  if (cost4 <= cost2 && cost4 <= cost3) return k4x2;
+  if (cost2 < cost3) return k2x2;
+  return 8 * ranges < split && split <= 9 * ranges ? k3x3 : k3x2;
+}
+
 template <int Format, int ABits, bool HalfOut, bool Partials>
 void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipStream_t stream) {
   const uint32_t batch = base_args.batch;
@@ -1547,48 +1601,7 @@ void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipSt
                   kDirectMaxWaves});
     hipLaunchKernelGGL(kernel, dim3(blocks * args.splits), dim3(64 * waves), lds, stream, args);
   };
-  // Row tiles per wave (R) and groups per load chunk (CH), by grid shape (measured on
-  // MI355X over the verifier's projections at 16 and 32 tokens, weights rotated past the
-  // Infinity Cache).  More tiles share each activation load and its expansion; shorter
-  // chunks need fewer registers, so more waves stay resident.  A split of one canonical
-  // range (the o and GDN out projections: 8-10 groups per split) runs one wave per
-  // workgroup and keeps one tile.  Grids below 1024 row tiles x splits take 2 tiles (2-group
-  // chunks at 17-32 tokens, 5-group chunks at 9-16; 3 tiles are slower at a short K, 8.8
-  // against 7.3 us for 880 row tiles x 18 groups).  Larger ones take the R of 2, 3, 4 whose
-  // fullest CU has the fewest row tiles, R ceil(workgroups / CUs): about all workgroups of
-  // such a grid are resident at once, so the launch lasts as long as that CU (W4 x 32
-  // tokens, 3 against 4 tiles: 1280 row tiles 14.9 / 16.9 us, 1728 row tiles 20.5 / 17.9,
-  // 4096 row tiles 40.5 / 37.9); within a thirtieth of each other the larger R (9496 row
-  // tiles 89.3 / 86.6).  Chunks are 2 groups; with 3 tiles 3 groups where a range has no
-  // more than nine (8.5 groups, W3 down projection: 13.4 against 14.7 us; 10 groups, 1030
-  // row tiles: 15.9 against 14.3).
-  const auto blocks_of = [&](unsigned r) {
-    uint64_t blocks = 0;
-    for (unsigned i = 0; i < 4; ++i) {
-      const bool used = i == 0 || base_args.tile_begin[i] != base_args.tile_begin[4];
-      if (used) blocks += (static_cast<uint64_t>(base_args.matrix[i].tiles) + r - 1) / r;
-    }
-    return blocks * base_args.splits;
-  };
-  const bool one_range = min_range_count(base_args.groups, base_args.splits) <= 1;
-  int shape;  // R x CH -- 1: 1 x 4, 2: 2 x 5, 3: 3 x 2, 4: 3 x 3, 5: 2 x 2, 6: 4 x 2
-  if (one_range) {
-    shape = 1;
-  } else if (blocks_of(1) < 4 * kComputeUnits) {
-    shape = batch > 16 ? 5 : 2;
-  } else {
-    unsigned best = 2;
-    uint64_t fullest = 2 * ((blocks_of(2) + kComputeUnits - 1) / kComputeUnits);
-    for (unsigned r = 3; r <= 4; ++r) {
-      const uint64_t tiles = r * ((blocks_of(r) + kComputeUnits - 1) / kComputeUnits);
-      if (tiles * 30 <= fullest * 31) {
-        best = r;
-        fullest = tiles;
-      }
-    }
-    const unsigned split = base_args.groups / base_args.splits;
-    shape = best == 2 ? 5 : (best == 4 ? 6 : (split <= 9 * range_count(split) ? 4 : 3));
-  }
+  const int shape = direct_shape(base_args);
   (void)total_tiles;
   if (batch <= 4) {
     go(lowbit_gemm_direct_kernel<Format, ABits, 4, 1, 3, 1, HalfOut, Partials>, 1, 1);
@@ -1596,22 +1609,22 @@ void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipSt
     go(lowbit_gemm_direct_kernel<Format, ABits, 2, 1, 6, 1, HalfOut, Partials>, 1, 1);
   } else if (batch <= 16) {
     switch (shape) {
-      case 2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 5, 2, HalfOut, Partials>, 2, 1); break;
-      case 3: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 3, HalfOut, Partials>, 3, 1); break;
-      case 4: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 3, 3, HalfOut, Partials>, 3, 1); break;
-      case 5: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 2, HalfOut, Partials>, 2, 1); break;
-      case 6: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 4, HalfOut, Partials>, 4, 1); break;
+      case k2x5: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 5, 2, HalfOut, Partials>, 2, 1); break;
+      case k3x2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 3, HalfOut, Partials>, 3, 1); break;
+      case k3x3: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 3, 3, HalfOut, Partials>, 3, 1); break;
+      case k2x2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 2, HalfOut, Partials>, 2, 1); break;
+      case k4x2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 2, 4, HalfOut, Partials>, 4, 1); break;
       default: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 1, 4, 1, HalfOut, Partials>, 1, 1); break;
     }
   } else if constexpr (ABits == 8) {
     go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 4, 1, HalfOut, Partials>, 1, 2);
   } else {
     switch (shape) {
-      case 2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 5, 2, HalfOut, Partials>, 2, 2); break;
-      case 3: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 3, HalfOut, Partials>, 3, 2); break;
-      case 4: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 3, 3, HalfOut, Partials>, 3, 2); break;
-      case 5: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 2, HalfOut, Partials>, 2, 2); break;
-      case 6: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 4, HalfOut, Partials>, 4, 2); break;
+      case k2x5: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 5, 2, HalfOut, Partials>, 2, 2); break;
+      case k3x2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 3, HalfOut, Partials>, 3, 2); break;
+      case k3x3: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 3, 3, HalfOut, Partials>, 3, 2); break;
+      case k2x2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 2, HalfOut, Partials>, 2, 2); break;
+      case k4x2: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 2, 4, HalfOut, Partials>, 4, 2); break;
       default: go(lowbit_gemm_direct_kernel<Format, ABits, 1, 2, 4, 1, HalfOut, Partials>, 1, 2); break;
     }
   }
@@ -2151,6 +2164,22 @@ extern "C" int32_t gfxinfer_debug_gemm_family(int32_t family, int32_t format, co
                     partials != nullptr ? nullptr : activation_scales, partials, columns, batch,
                     half_output != 0, static_cast<hipStream_t>(stream), argmax_keys, argmax_rows, splits,
                     family);
+}
+
+extern "C" int32_t gfxinfer_debug_gemm_direct_shape(size_t rows, size_t columns, uint32_t batch, uint32_t splits) {
+  if (rows == 0 || rows % 16 != 0 || rows / 16 > (1u << 28) || columns == 0 || columns % kGroup != 0 ||
+      columns > (1u << 30) || batch < 9 || batch > 32 || splits == 0 || splits > kMaxSplits ||
+      splits > columns / kGroup) {
+    return 0;
+  }
+  GemmArgs args{};
+  args.matrix[0].tiles = static_cast<uint32_t>(rows / 16);
+  for (unsigned i = 1; i < 5; ++i) args.tile_begin[i] = args.matrix[0].tiles;
+  args.groups = static_cast<uint32_t>(columns / kGroup);
+  args.batch = batch;
+  args.splits = splits;
+  constexpr int32_t kShapes[] = {0, 104, 205, 302, 303, 202, 402};
+  return kShapes[direct_shape(args)];
 }
 
 extern "C" int32_t gfxinfer_launch_lowbit_row_gather_tiled(int32_t format,

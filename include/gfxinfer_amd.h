@@ -202,6 +202,11 @@ int32_t gfxinfer_debug_gemm_partials(int32_t format, const uint8_t* tiled_weight
                                      size_t rows, size_t columns, uint32_t batch,
                                      int32_t* partials, void* stream);
 
+/* Test hook, no reference counterpart, host only: the shape the launchers above pick for one
+ * A4 matrix at 9-32 tokens, 100 x row tiles per wave + groups per load chunk (0: not a shape
+ * they take). */
+int32_t gfxinfer_debug_gemm_direct_shape(size_t rows, size_t columns, uint32_t batch, uint32_t splits);
+
 /* Test and bench hook, no reference counterpart: one A4 GEMM launch through a named
  * kernel family, 1 = the MFMA kernels (16x16x64 int8, used for every shape by the
  * launchers above) or 2 = the v_dot8_i32_i4 kernel (W3/W4, 1-8 tokens, activation

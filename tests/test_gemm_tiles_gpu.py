@@ -8,15 +8,31 @@ import pytest
 
 from gpu_util import say
 
-pytestmark = pytest.mark.gpu
+# format, row tiles, columns, splits, tokens, the shape the launcher takes (100 x row tiles per wave + groups per chunk):
+# last blocks of every length, 2 to 14 ranges on up to eight waves (17408 columns: some waves take two ranges)
+CASES = [
+    (2, 1024, 1408, 1, 9, 205), (3, 1601, 1408, 1, 17, 202), (1, 1601, 1536, 1, 32, 202), (2, 1100, 2560, 1, 16, 205),
+    (3, 1538, 1408, 1, 32, 202), (2, 1026, 2816, 2, 24, 302), (3, 1280, 2304, 1, 11, 205), (2, 9217, 1408, 1, 20, 402),
+    (3, 1283, 1408, 1, 30, 205), (2, 2401, 1408, 1, 12, 202), (3, 2399, 1408, 1, 32, 202), (2, 1100, 5120, 1, 32, 302),
+    (3, 1027, 4352, 2, 13, 303), (2, 1028, 4352, 2, 19, 303), (3, 2049, 3072, 1, 10, 302), (2, 1726, 5120, 1, 16, 402),
+    (3, 1725, 5120, 1, 21, 402), (2, 1024, 17408, 1, 32, 402), (3, 1023, 17408, 1, 31, 202), (2, 1027, 17408, 1, 15, 302),
+    (3, 1100, 17408, 1, 32, 302), (1, 3070, 4096, 1, 9, 402)]
 
 
-# row tiles: 1024 and 1601 take 4 (1601 with a last block of one tile), 1100 and 1538 take 3,
-# 1026 x 2 splits takes 3 with 3-group chunks, 1280 takes 2 or 3, 9217 takes 4 by the tie rule
-@pytest.mark.parametrize("fmt,tiles,cols,splits,tokens", [
-    (2, 1024, 1408, 1, 9), (3, 1601, 1408, 1, 17), (1, 1601, 1536, 1, 32), (2, 1100, 2560, 1, 16),
-    (3, 1538, 1408, 1, 32), (2, 1026, 2816, 2, 24), (3, 1280, 2304, 1, 11), (2, 9217, 1408, 1, 20)])
-def test_row_tiles_per_wave(gx, device, fmt, tiles, cols, splits, tokens):
+@pytest.mark.parametrize("fmt,tiles,cols,splits,tokens,shape", CASES)
+def test_shape_of_a_case(gx, fmt, tiles, cols, splits, tokens, shape):
+    assert gx.lib().gfxinfer_debug_gemm_direct_shape(tiles * 16, cols, tokens, splits) == shape
+
+
+def test_cases_take_every_shape(gx):
+    for lo, hi in ((9, 16), (17, 32)):
+        assert {c[5] for c in CASES if lo <= c[4] <= hi} == {202, 205, 302, 303, 402}
+    assert gx.lib().gfxinfer_debug_gemm_direct_shape(5120, 1280, 32, 1) == 104   # one range
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,tiles,cols,splits,tokens,shape", CASES)
+def test_row_tiles_per_wave(gx, device, fmt, tiles, cols, splits, tokens, shape):
     import torch
     rows = tiles * 16
     g = torch.Generator(device=device).manual_seed(tiles + tokens)
