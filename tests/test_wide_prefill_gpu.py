@@ -26,10 +26,11 @@ def _problem(gx, orc, fmt, rows, cols, tokens, seed):
 
 
 # Edges of the 128 x 128 block and of a 16-token tile, one and several ranges and splits,
-# fewer and more steps than LDS stages, a short last row block.
+# fewer and more steps than LDS stages, a short last row block; the reference's longest K in its planes.
 @pytest.mark.parametrize("fmt,rows,cols,tokens,splits", [
     (3, 16, 128, 1, 1), (2, 128, 256, 16, 1), (1, 144, 384, 33, 1), (3, 272, 1280, 128, 1), (2, 112, 1408, 129, 1),
-    (3, 256, 2688, 65, 2), (2, 160, 5120, 100, 4), (1, 16, 2560, 257, 8), (2, 128, 640, 47, 5)])
+    (3, 256, 2688, 65, 2), (2, 160, 5120, 100, 4), (1, 16, 2560, 257, 8), (2, 128, 640, 47, 5),
+    (3, 272, 17408, 97, 4), (2, 144, 5120, 200, 1)])
 def test_prefill_gemm_equals_canonical_sum(gx, orc, device, fmt, rows, cols, tokens, splits):
     import torch
     codes, scales, tiled, tscales, packed, ascales = _problem(gx, orc, fmt, rows, cols, tokens, rows + cols + tokens)
@@ -78,7 +79,7 @@ def _blocks(session, prompt, mtp):
     return token
 
 
-def _same(a, b, rows):
+def _same(a, b, rows, context=CONTEXT):
     assert (a.position(), a.mtp_position()) == (b.position(), b.mtp_position())
     spec = a.model.spec
     kv = spec.kv_head_count * spec.attention_head_size
@@ -86,7 +87,7 @@ def _same(a, b, rows):
         x, y = a.buffer(name, dtype), b.buffer(name, dtype)
         if "cache" in name:
             used = a.mtp_position() if name.startswith("mtp") else a.position()
-            x, y = (v.reshape(-1, CONTEXT, kv)[:, :used] for v in (x, y))
+            x, y = (v.reshape(-1, context, kv)[:, :used] for v in (x, y))
         assert np.array_equal(x, y), name
     x, y = (s.buffer("logits", np.uint32, rows * spec.vocabulary_size) for s in (a, b))
     assert np.array_equal(x, y)
@@ -185,3 +186,27 @@ def test_prompt_without_scratch_runs_in_blocks(model):
     _same(a, b, 5)
     a.close()
     b.close()
+
+
+# Four layers (three GDN, one attention) at real widths.  The attention of a pass runs in several launches here: at
+# 40/8 x 128 with its partial results in the scratch (context 4096) and in the block workspace (8192), and at 24/4 x 256.
+@pytest.mark.parametrize("shape,n,context", [("27b", 2600, 4096), ("27b", 1100, 8192), ("reference", 1125, 2048)])
+def test_full_width_wide_prefill_equals_blocks(device, shape, n, context):
+    from gfxinfer_amd import runtime as rt
+    spec = rt.qwen38_27b_spec() if shape == "27b" else rt.qwen38_reference_spec()
+    spec.layer_count, spec.w3_mlp_layers = 4, 3
+    say("full-width model", shape)
+    model = rt.SyntheticModel(spec, 23)
+    prompt = np.random.default_rng(n).integers(0, spec.tokenizer_vocabulary_size, n).astype(np.uint32)
+    a, b = (rt.QwenDecodeSession(model, context, 0, keep_logits=True) for _ in range(2))
+    say("blocks", shape, n)
+    want = _blocks(a, prompt, True)
+    say("wide passes", shape, n)
+    assert b.prefill(prompt) == want
+    _same(a, b, (n - 1) % 32 + 1, context)
+    ra, rb = a.speculative_step(want, 4), b.speculative_step(want, 4)
+    assert (ra.tokens, ra.accepted_drafts) == (rb.tokens, rb.accepted_drafts)
+    _same(a, b, 5, context)
+    a.close()
+    b.close()
+    model.close()
