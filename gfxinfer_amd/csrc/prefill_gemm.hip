@@ -119,7 +119,8 @@ __global__ __launch_bounds__(256) void prefill_expand_kernel(const uint8_t* __re
 }
 
 // ---------------------------------------------------------------------------
-// GEMM.  Workgroup = WR x WT waves, wave = RT row tiles x CT token tiles of 16 x 16.
+// GEMM.  Workgroup = WR x WT waves, wave = RT row tiles x CT token tiles of 16 x 16: 128 rows
+// x 128 tokens.
 // One group of K per step.  The token side arrives by DMA (buffer_load ... lds) in operand
 // order, three steps ahead through four LDS stages; the row side is loaded into one of
 // two register sets three steps ahead and widened one step ahead, each wave an equal share
@@ -139,7 +140,10 @@ struct PrefillArgs {
   uint32_t token_blocks;
 };
 
-template <int Format, bool HalfOut, int RT, int CT, int WR, int WT>
+constexpr int RT = 4, CT = 4;       // 16-row / 16-token tiles of a wave
+constexpr unsigned WR = 2, WT = 2;  // waves of a workgroup
+
+template <int Format, bool HalfOut>
 __global__ __launch_bounds__(64 * WR * WT, 2) void prefill_gemm_kernel(PrefillArgs args) {
   constexpr unsigned LB = lane_bytes(Format), WD = LB / 4;
   constexpr unsigned kRows = WR * RT, kCols = WT * CT, kWaves = WR * WT;  // 16-row / 16-token tiles
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void prefill_gemm_kernel(PrefillAr
   constexpr unsigned kMetaDma = (kCols + 2 * kWaves - 1) / (2 * kWaves);  // 64 x 4-byte pieces of the meta rows per wave
   constexpr unsigned kTokenLoads = kDma + kMetaDma;    // vector-memory instructions of load_tokens
   constexpr unsigned kLoads = kOwn + 1;            // ... and of load_weights
-  static_assert(kRows % kWaves == 0 && RT == 4 && CT == 4 && kOwn * 16 <= 64, "tile shape");
+  static_assert(kRows % kWaves == 0 && kOwn == 2 && CT == 4, "two row tiles widened between four token tiles");
   constexpr unsigned kOut = 0x80000000u;
   __shared__ __align__(16) uint8_t row_side[2][kRows * kFragmentBytes];
   // One object per stage, so that the compiler sees which DMA a read can meet: from one
@@ -344,11 +348,10 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void prefill_gemm_kernel(PrefillAr
     // The next group's tiles are widened between the token tiles, in the shadow of their
     // matrix instructions (before the first token tile: 3 to 6 % slower at every shape,
     // W3 34816 x 5120 x 512 tokens 149 us against 142, W3 12288 x 5120 59.7 against 56).
-    static_assert(kOwn <= 2 && CT == 4, "widening spread over the token tiles");
     token_tile(std::integral_constant<int, 0>{});
     widen_tile(0, buf ^ 1u, wregs[buf ^ 1u]);
     token_tile(std::integral_constant<int, 1>{});
-    if constexpr (kOwn > 1) widen_tile(1, buf ^ 1u, wregs[buf ^ 1u]);
+    widen_tile(1, buf ^ 1u, wregs[buf ^ 1u]);
     token_tile(std::integral_constant<int, 2>{});
     widen_scales(buf ^ 1u, sregs[buf ^ 1u]);
     load_weights(g + 3u, wregs[buf ^ 1u], sregs[buf ^ 1u]);
@@ -403,19 +406,16 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void prefill_gemm_kernel(PrefillAr
 }
 
 template <int Format, bool HalfOut>
-void launch(const PrefillArgs& base, hipStream_t stream) {
-  auto go = [&](auto kernel, unsigned row_tiles, unsigned token_tiles, unsigned threads) {
-    PrefillArgs args = base;
-    uint32_t units = 0;
-    for (unsigned i = 0; i < 4; ++i) {
-      args.unit_begin[i] = units;
-      if (args.matrix[i].weights != nullptr) units += (args.matrix[i].tiles + row_tiles - 1) / row_tiles * args.splits;
-    }
-    args.unit_begin[4] = units;
-    args.token_blocks = (args.tiles + token_tiles - 1) / token_tiles;
-    hipLaunchKernelGGL(kernel, dim3((units + 7) / 8 * 8 * args.token_blocks), dim3(threads), 0, stream, args);
-  };
-  go(prefill_gemm_kernel<Format, HalfOut, 4, 4, 2, 2>, 8, 8, 256);
+void launch(PrefillArgs& args, hipStream_t stream) {
+  uint32_t units = 0;
+  for (unsigned i = 0; i < 4; ++i) {
+    args.unit_begin[i] = units;
+    if (args.matrix[i].weights != nullptr) units += (args.matrix[i].tiles + WR * RT - 1) / (WR * RT) * args.splits;
+  }
+  args.unit_begin[4] = units;
+  args.token_blocks = (args.tiles + WT * CT - 1) / (WT * CT);
+  hipLaunchKernelGGL((prefill_gemm_kernel<Format, HalfOut>), dim3((units + 7) / 8 * 8 * args.token_blocks),
+                     dim3(64 * WR * WT), 0, stream, args);
 }
 
 }  // namespace
