@@ -663,8 +663,8 @@ def reference_bench_rates(model, spec, block_sizes=(5, 32), blocks=12, mtp_steps
 def prefill_bench(prompt_tokens=512, serial_tokens=64, seed=2026, context=4096):
     """Chunked prefill against the reference's serial prefill loop on the synthetic
     27B-shaped model: time to the first generated token for a `prompt_tokens` prompt
-    with the MTP cache kept in step (gfxinfer_session_prefill, 32-token verifier blocks
-    + batched MTP cache update), and the per-token rate of the loop the reference CLI
+    with the MTP cache kept in step (gfxinfer_session_prefill: wide passes from 65 tokens
+    on, 32-token verifier blocks below), and the per-token rate of the loop the reference CLI
     runs (greedy_step + mtp_draft per prompt token, cli/main.cpp:1055-1069), timed over
     `serial_tokens` tokens.  Both leave the same state (tests/test_prefill_generate_gpu.py)."""
     import numpy as np
@@ -677,7 +677,7 @@ def prefill_bench(prompt_tokens=512, serial_tokens=64, seed=2026, context=4096):
     prompt = [int(t) for t in prompt]
     try:
         chunked = QwenDecodeSession(model, context, 0)
-        chunked.prefill(prompt[:64])  # warm-up of the block kernels
+        chunked.prefill(prompt)  # warm-up: kernels loaded, the model's scratch allocated
         chunked.close()
         chunked = QwenDecodeSession(model, context, 0)
         torch.cuda.synchronize()
@@ -817,7 +817,7 @@ def pmc_probe(launches=8, rows=17408, cols=5120, batch=5):
 
 def headline_kernel_digest():
     """SHA-256 (first 16 hex digits) of the headline kernel's source: lowbit_gemv.hip from
-    its operand expansion through lowbit_gemm_kernel, plus common.hpp.  A committed
+    its operand expansion through lowbit_gemm_kernel, gemm_common.hpp and common.hpp.  A committed
     profile records the digest of the source it measured, so a changed kernel shows up
     as a stale profile instead of passing its old counters on."""
     import hashlib
@@ -825,7 +825,8 @@ def headline_kernel_digest():
     text = open(os.path.join(csrc, "lowbit_gemv.hip")).read()
     begin, end = text.index("// Operand expansion."), text.index("// Direct-operand GEMM.")
     digest = hashlib.sha256(text[begin:end].encode())
-    digest.update(open(os.path.join(csrc, "common.hpp"), "rb").read())
+    for header in ("gemm_common.hpp", "common.hpp"):
+        digest.update(open(os.path.join(csrc, header), "rb").read())
     return digest.hexdigest()[:16]
 
 
