@@ -346,8 +346,9 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void prefill_gemm_kernel(PrefillAr
         for (int i = 0; i < 4; ++i) acc[r][t][i] = fmaf(c[r][i], scale[4 * r + i], acc[r][t][i]);
     };
     // The next group's tiles are widened between the token tiles, in the shadow of their
-    // matrix instructions (before the first token tile: 3 to 6 % slower at every shape,
-    // W3 34816 x 5120 x 512 tokens 149 us against 142, W3 12288 x 5120 59.7 against 56).
+    // matrix instructions (before the first token tile, with the expansion: W3 34816 x 5120 x
+    // 512 tokens 158 us against 149, W3 12288 x 5120 64.7 against 63, W3 5120 x 17408 in four
+    // planes 90.7 against 85, W4 5120 x 5120 36.4 against 34.0).
     token_tile(std::integral_constant<int, 0>{});
     widen_tile(0, buf ^ 1u, wregs[buf ^ 1u]);
     token_tile(std::integral_constant<int, 1>{});

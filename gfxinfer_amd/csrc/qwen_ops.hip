@@ -1248,11 +1248,16 @@ __global__ __launch_bounds__(256) void gdn_restore_conv_kernel(
 // a row, four times over: a token costs it one read each of the deltas, the decay and the
 // keys per four pieces (reads per piece made the LDS the bound), and the four quarters of
 // the state, one after the other, overlap their stores with the next one's arithmetic.
-// Streamed: the states are stored past the caches.  States of all layers that do not stay
-// in the last-level cache until they are next read come from HBM again either way, and
-// their stores then cost the loads of the same launch less (48 layers x 48 heads, three
-// sets in turn, 19 tokens: 93 -> 76 us, one token 67 -> 53 us; x 32 heads, 100 MB, 61 -> 51);
-// at 50 MB and one token, where they do stay, the plain stores win (18.1 against 19.2 us).
+// Streamed: the states are stored past the caches, above 64 MB of them.  Three sets of
+// states in turn, plain against streamed: 48 layers x 48 heads (151 MB) 19 tokens 88 -> 73 us,
+// one token 66 -> 52; x 32 heads (101 MB) 53 -> 49 and 40 -> 36; 75 MB 43 -> 40, but one token
+// 26 -> 28; 50 MB and one token, where all sets stay in the last-level cache, 17.5 -> 19.1.
+// In a session gigabytes of weights pass before the states are read again, and what plain
+// stores leave in the caches slows the reads after them: restore and the read of 1 GB that
+// follows, 151 MB 297 -> 281 us (one token 272 -> 268), 75 MB 258 -> 246 (238 -> 236), 67 MB
+// 246 -> 234 (232 -> 232), 50 MB 238 -> 229 (226 -> 223), 34 MB 226 -> 224 (214 -> 215), 13 MB
+// no difference.  So below the line streaming would pay in a session too from about 50 MB on,
+// and costs where the launch runs back to back; the models here have 101 and 151 MB.
 constexpr unsigned kRestoreThreads = 256;
 constexpr std::size_t kRestoreStreamed = std::size_t{64} << 20;
 

@@ -37,7 +37,9 @@ constexpr std::size_t kMaxPlanes = 8;  // split-K planes of a projection (GEMM e
 // once per 128 tokens and launches each layer's kernels once, whatever its length.
 constexpr std::size_t kWideTokens = 512;
 // Fewer tokens than this go in 32-token blocks: up to two blocks are faster than one wide
-// pass (27B shape: 12.1 against 13.5 ms at 64 tokens, 17.0 against 14.4 ms at 80).
+// pass, three are not (64 layers, blocks against wide pass, 33 / 64 / 65 / 80 tokens: 27B shape
+// 10.0 / 11.6 / 15.6 / 16.3 against 11.7 / 12.3 / 12.4 / 12.7 ms, the reference's heads
+// 10.8 / 12.6 / 17.0 / 17.8 against 12.2 / 12.9 / 12.9 / 13.3 ms).
 constexpr std::size_t kWideMinimum = 65;
 
 struct Matrix {
