@@ -666,7 +666,7 @@ def prefill_bench(prompt_tokens=512, serial_tokens=64, seed=2026, context=4096):
     with the MTP cache kept in step (gfxinfer_session_prefill: wide passes from 65 tokens
     on, 32-token verifier blocks below), and the per-token rate of the loop the reference CLI
     runs (greedy_step + mtp_draft per prompt token, cli/main.cpp:1055-1069), timed over
-    `serial_tokens` tokens.  Both leave the same state (tests/test_prefill_generate_gpu.py)."""
+    `serial_tokens` tokens (0: not run).  Both leave the same state (tests/test_prefill_generate_gpu.py)."""
     import numpy as np
     import torch
     from gfxinfer_amd.runtime import QwenDecodeSession, SyntheticModel, qwen38_27b_spec
@@ -685,21 +685,22 @@ def prefill_bench(prompt_tokens=512, serial_tokens=64, seed=2026, context=4096):
         chunked.prefill(prompt)
         chunked_s = time.perf_counter() - t0
         chunked.close()
-        serial = QwenDecodeSession(model, context, 0)
-        serial.greedy_step(prompt[0])
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for t in prompt[1:1 + serial_tokens]:
-            serial.mtp_draft(t)
-            serial.greedy_step(t)
-        serial_s = time.perf_counter() - t0
-        serial.close()
+        line = {"prefill": "chunked", "prompt_tokens": prompt_tokens, "seconds": round(chunked_s, 4),
+                "tok_s": round(prompt_tokens / chunked_s, 1)}
+        if serial_tokens:
+            serial = QwenDecodeSession(model, context, 0)
+            serial.greedy_step(prompt[0])
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for t in prompt[1:1 + serial_tokens]:
+                serial.mtp_draft(t)
+                serial.greedy_step(t)
+            serial_s = time.perf_counter() - t0
+            serial.close()
+            line["serial_tok_s"] = round(serial_tokens / serial_s, 1)
+            line["speedup"] = round((prompt_tokens / chunked_s) / (serial_tokens / serial_s), 2)
     finally:
         model.close()
-    line = {"prefill": "chunked", "prompt_tokens": prompt_tokens, "seconds": round(chunked_s, 4),
-            "tok_s": round(prompt_tokens / chunked_s, 1),
-            "serial_tok_s": round(serial_tokens / serial_s, 1),
-            "speedup": round((prompt_tokens / chunked_s) / (serial_tokens / serial_s), 2)}
     print(json.dumps(line), flush=True)
     return line
 
@@ -868,7 +869,7 @@ def main():
     ap.add_argument("--verify-rounds", type=int, default=60)
     ap.add_argument("--no-reference-rates", action="store_true",
                     help="skip the verifier-only block_step and proposal-only rates (a round profile "
-                         "then ends with the last round)")
+                         "then ends with the last round), and with --prefill the serial loop")
     ap.add_argument("--verify-model", choices=("27b", "reference"), default="27b",
                     help="verify-round model heads: the BASELINE 27B shape or the reference's own model")
     ap.add_argument("--long-context", type=int, default=3584,
@@ -928,7 +929,7 @@ def main():
         read_floor_bench()
         return
     if args.prefill:
-        prefill_bench()
+        prefill_bench(serial_tokens=0 if args.no_reference_rates else 64)
         return
 
     r = gemv_bench(args.steps, args.warmup)
