@@ -73,7 +73,7 @@ SIGNATURES: dict[str, tuple] = {
     "gfxinfer_launch_gfx950_i4_gemm_argmax_no_alloc": (I32, [I32, P, P, P, P, P, SZ, SZ, U32, SZ, P, P, P]),
     "gfxinfer_debug_gemm_partials": (I32, [I32, P, I32, P, SZ, SZ, U32, P, P]),
     "gfxinfer_debug_gemm_family": (I32, [I32, I32, P, P, P, P, P, I32, P, P, U32, SZ, SZ, U32, U32, P]),
-    "gfxinfer_debug_gemm_direct_shape": (I32, [SZ, SZ, U32, U32]),
+    "gfxinfer_debug_gemm_direct_shape": (I32, [I32, SZ, SZ, U32, U32]),
     "gfxinfer_debug_gemm_prefill_workspace_bytes": (SZ, [SZ, U32]),
     "gfxinfer_debug_gemm_prefill": (I32, [I32, P, P, P, P, P, I32, SZ, SZ, U32, U32, P, SZ, P]),
     "gfxinfer_debug_stream_read": (I32, [P, SZ, P, U32, P]),

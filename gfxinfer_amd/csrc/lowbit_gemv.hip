@@ -1540,9 +1540,11 @@ unsigned choose_waves(uint32_t groups) {
 //     1100 row tiles 16.4 / 14.8 / 16.6 us, 1728 21.1 / 21.0 / 18.3, 2560 28.3 / 26.7 / 25.7,
 //     9496 92.5 / 88.1 / 84.8; x 80 groups, eight waves that hold a CU alone: 2560 49.1 /
 //     48.9 / 49.3; 12 tokens x 40 groups: 1100 12.0 / 11.8 / 13.4, 2560 19.9 / 21.7 / 21.4,
-//     9496 69.8 / 71.0 / 68.9).  More than 2560 row tiles x 80 groups, which no model here
+//     9496 69.8 / 71.0 / 68.9).  With A8 activations, twice the bytes to share, 0.86 and 0.80
+//     (W4 x 16 tokens x 40 groups: 1280 16.9 / 14.6 / 16.5, 2048 21.2 / 20.9 / 18.4, 2560
+//     25.8 / 25.6 / 24.6).  More than 2560 row tiles x 80 groups, which no model here
 //     has, can miss the best by 7 % (3300 x 32 tokens W3: 57.9 us, 54.1 with 3 tiles).
-//   * Up to three ranges a workgroup is two or three waves, several share a CU, and the
+//   * Up to three ranges (A8: two) a workgroup is two or three waves, several share a CU, and the
 //     launch is as long as one of them: while the fullest CU holds no more than four
 //     workgroups of 2 tiles, those (1728 row tiles, 18 groups, W3: 32 tokens 11.2 us against
 //     13.5 with 4 tiles, 12 tokens 9.0 against 10.4), in 5-group chunks where a range is two
@@ -1553,7 +1555,7 @@ unsigned choose_waves(uint32_t groups) {
 //     16.8; 10 groups, 1100 row tiles: 14.8 against 16.4).
 enum DirectShape : int { k1x4 = 1, k2x5, k3x2, k3x3, k2x2, k4x2 };  // R x CH
 
-int direct_shape(const GemmArgs& args) {
+int direct_shape(const GemmArgs& args, int abits) {
   if (min_range_count(args.groups, args.splits) <= 1) return k1x4;
   const auto blocks_of = [&](unsigned r) {
     uint64_t blocks = 0;
@@ -1569,8 +1571,10 @@ int direct_shape(const GemmArgs& args) {
   const auto fullest = [&](unsigned r) { return r * ((blocks_of(r) + kComputeUnits - 1) / kComputeUnits); };
   const unsigned split = args.groups / args.splits, ranges = range_count(split);
   const uint64_t tiles2 = fullest(2);
-  if (ranges <= 3 && tiles2 <= 8) return ranges <= 2 && tiles2 <= 6 ? k2x5 : k2x2;
-  const uint64_t cost2 = tiles2 * 100, cost3 = fullest(3) * 95, cost4 = fullest(4) * (two_blocks && ranges >= 4 && ranges < 8 ? 83 : 90);
+  if (ranges <= (abits == 8 ? 2u : 3u) && tiles2 <= 8) return ranges <= 2 && tiles2 <= 6 ? k2x5 : k2x2;
+  const unsigned each3 = abits == 8 ? 86 : 95;
+  const unsigned each4 = abits == 8 ? 80 : (two_blocks && ranges >= 4 && ranges < 8 ? 83 : 90);
+  const uint64_t cost2 = tiles2 * 100, cost3 = fullest(3) * each3, cost4 = fullest(4) * each4;
   if (cost4 <= cost2 && cost4 <= cost3) return k4x2;
   if (cost2 < cost3) return k2x2;
   return 8 * ranges < split && split <= 9 * ranges ? k3x3 : k3x2;
@@ -1601,7 +1605,7 @@ void launch_direct_kernel(const GemmArgs& base_args, uint32_t total_tiles, hipSt
                   kDirectMaxWaves});
     hipLaunchKernelGGL(kernel, dim3(blocks * args.splits), dim3(64 * waves), lds, stream, args);
   };
-  const int shape = direct_shape(base_args);
+  const int shape = direct_shape(base_args, ABits);
   (void)total_tiles;
   if (batch <= 4) {
     go(lowbit_gemm_direct_kernel<Format, ABits, 4, 1, 3, 1, HalfOut, Partials>, 1, 1);
@@ -2166,9 +2170,10 @@ extern "C" int32_t gfxinfer_debug_gemm_family(int32_t family, int32_t format, co
                     family);
 }
 
-extern "C" int32_t gfxinfer_debug_gemm_direct_shape(size_t rows, size_t columns, uint32_t batch, uint32_t splits) {
-  if (rows == 0 || rows % 16 != 0 || rows / 16 > (1u << 28) || columns == 0 || columns % kGroup != 0 ||
-      columns > (1u << 30) || batch < 9 || batch > 32 || splits == 0 || splits > kMaxSplits ||
+extern "C" int32_t gfxinfer_debug_gemm_direct_shape(int32_t activation_bits, size_t rows, size_t columns,
+                                                    uint32_t batch, uint32_t splits) {
+  if ((activation_bits != 4 && activation_bits != 8) || batch > (activation_bits == 8 ? 16u : 32u) || rows == 0 || rows % 16 != 0 || rows / 16 > (1u << 28) || columns == 0 || columns % kGroup != 0 ||
+      columns > (1u << 30) || batch < 9 || splits == 0 || splits > kMaxSplits ||
       splits > columns / kGroup) {
     return 0;
   }
@@ -2179,7 +2184,7 @@ extern "C" int32_t gfxinfer_debug_gemm_direct_shape(size_t rows, size_t columns,
   args.batch = batch;
   args.splits = splits;
   constexpr int32_t kShapes[] = {0, 104, 205, 302, 303, 202, 402};
-  return kShapes[direct_shape(args)];
+  return kShapes[direct_shape(args, activation_bits)];
 }
 
 extern "C" int32_t gfxinfer_launch_lowbit_row_gather_tiled(int32_t format,

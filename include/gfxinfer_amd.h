@@ -203,9 +203,10 @@ int32_t gfxinfer_debug_gemm_partials(int32_t format, const uint8_t* tiled_weight
                                      int32_t* partials, void* stream);
 
 /* Test hook, no reference counterpart, host only: the shape the launchers above pick for one
- * A4 matrix at 9-32 tokens, 100 x row tiles per wave + groups per load chunk (0: not a shape
- * they take). */
-int32_t gfxinfer_debug_gemm_direct_shape(size_t rows, size_t columns, uint32_t batch, uint32_t splits);
+ * matrix at 9-32 tokens (A8: 9-16), 100 x row tiles per wave + groups per load chunk (0: no
+ * such launch). */
+int32_t gfxinfer_debug_gemm_direct_shape(int32_t activation_bits, size_t rows, size_t columns,
+                                         uint32_t batch, uint32_t splits);
 
 /* Test and bench hook, no reference counterpart: one A4 GEMM launch through a named
  * kernel family, 1 = the MFMA kernels (16x16x64 int8, used for every shape by the
